@@ -40,6 +40,7 @@
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define PF_NT 256
 
@@ -428,6 +429,413 @@ GH_GEMM_W8_FMT(q8, Q8W)
 GH_GEMM_W8_FMT(bf16, Bf16W)
 GH_GEMM_PAIR_W8(gh_pf_gateup_q4_m128_n64, Q4W, 128, 64, 1, true, _s_w8)
 
+// ---------------------------------------------------------------------------
+// The wide tile GEMM: one 512-thread workgroup per CU owns 64 TM tokens by BR
+// (256 or 128) weight rows (for a gate/up pair half of them of each matrix),
+// 2 x 4 wavefronts of (32 TM) x (BR / 4) on v_mfma_f32_16x16x32_f16 (or
+// _bf16).  Operands as the tile GEMM's above; a block's sum is its hi
+// products, then its lo products (the streamed GEMM's order below).
+//
+// What bounds it: the matrix pipes and the power they draw.  A step of one
+// block of K is 2048 matrix cycles of a CU at TM = 4, BR = 256, and about
+// 1570 vector cycles (a scale FMA per result, the weights' unpacking); under
+// random data the chip runs these at 1.4-1.8 GHz (a register-only loop of the
+// same MFMA: 1.9-2.0 PFLOP/s, 1.65-1.85 for the 32x32x16 form, which is why
+// this one uses 16x16x32), so whatever else a step does costs time as power
+// even where it overlaps:
+//  * operands go from memory to LDS directly (16 bytes per lane, no registers
+//    and no LDS store instructions).  The A rows are swizzled on the way, by
+//    permuting the lanes' source addresses within a row's 128 bytes, so that
+//    the operand reads are free of bank conflicts;
+//  * quantized weights stay packed in LDS, four blocks of K (80 or 144 bytes
+//    of a row) at a time, and each wavefront unpacks the words of its rows as
+//    it reads them: a quarter (Q4) of the LDS bytes of fp16 weights;
+//  * one barrier per step, ahead of the last 16 rows, whose MFMAs then cover
+//    the next step's first LDS reads; two to four steps of A in flight.
+// The waits are written out (vmcnt counts the loads issued since), because the
+// compiler would wait for every load to LDS before any LDS read.
+//
+// Measured, 12B gate/up of 512 tokens (activation split included): Q4 309 ->
+// 207 us (1170 TFLOP/s executed), Q8 315 -> 218, bf16 338 -> 187; without its
+// loads the Q4 form takes 200 of 225 us, without the LDS reads of A as well
+// 176.  The gate/up of 128 tokens (TM 2, BR 128, which keeps K unsplit) 91 ->
+// 70 us, of 64 tokens 64 -> 53 us.
+// ---------------------------------------------------------------------------
+#define PF_WIDE_NT 512
+
+// 16 bytes per lane from src to LDS byte lds + 16 * lane.
+__device__ __forceinline__ void load_lds16(const void* src, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src),
+               "s"(lds)
+               : "memory");
+}
+__device__ __forceinline__ void load_lds16(uint32_t off, const void* base, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off),
+               "s"(base), "s"(lds)
+               : "memory");
+}
+template <int N>
+__device__ __forceinline__ void wait_loads_barrier() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+// A weight format of the wide tile.  Quantized: kChunks 16-byte pieces of a
+// row hold four blocks, and per(rows, j) pieces per thread of a group of four
+// blocks are loaded in step j of the four.  bf16: a step's 64 bytes of a row (4 pieces, swizzled), two per thread.
+// raw: one block of one row as a lane's operand needs it (elements 8 g ..
+// 8 g + 7, g = lane / 16); pair: two of the operand's eight halves.
+struct WQ4 {
+  static constexpr bool kBf16 = false;
+  static constexpr int kChunks = 5, kRaw = 1;
+  static constexpr int per(int rows, int j) { return j == 0 ? rows / 128 : j == 1; }
+  __device__ static void raw(const uint8_t* row, uint32_t g, uint32_t* w, float* d) {
+    const uint32_t* p = reinterpret_cast<const uint32_t*>(row);
+    *d = __uint_as_float(p[0]);
+    w[0] = p[1 + g];
+  }
+  // the operand's pair p, as Q4W::ints (mask and magic: see wide_tile)
+  __device__ static uint32_t pair(const uint32_t* w, int p, uint32_t mask, uint32_t magic) {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    uint32_t pr;
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(pr) : "v"(w[0] >> (4 * p)), "v"(mask), "s"(magic));
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, pr) + h2{(_Float16)-1032.0f, (_Float16)-1032.0f});
+  }
+};
+struct WQ8 {
+  static constexpr bool kBf16 = false;
+  static constexpr int kChunks = 9, kRaw = 2;
+  static constexpr int per(int rows, int j) { return j < 2 ? (rows == 256 ? 3 : 2) - j : 0; }
+  __device__ static void raw(const uint8_t* row, uint32_t g, uint32_t* w, float* d) {
+    const uint32_t* p = reinterpret_cast<const uint32_t*>(row);
+    *d = __uint_as_float(p[0]);
+    w[0] = p[1 + 2 * g];
+    w[1] = p[2 + 2 * g];
+  }
+  // byte q + 128 under the exponent of 1024 is 1024 + (q + 128), exactly; the
+  // packed add of -1152 leaves q
+  __device__ static uint32_t pair(const uint32_t* w, int p, uint32_t, uint32_t magic) {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    const uint32_t u = __builtin_amdgcn_perm(magic, w[p / 2] ^ 0x80808080u, p % 2 ? 0x07030702u : 0x07010700u);
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, u) + h2{(_Float16)-1152.0f, (_Float16)-1152.0f});
+  }
+};
+struct WBf16 {
+  static constexpr bool kBf16 = true;
+  static constexpr int kChunks = 4, kRaw = 4;
+  static constexpr int per(int rows, int) { return rows / 128; }
+  __device__ static void raw(const uint8_t* chunk, uint32_t, uint32_t* w, float*) {
+    const u32x4 v = *reinterpret_cast<const u32x4*>(chunk);
+#pragma unroll
+    for (int k = 0; k < 4; k++) w[k] = v[k];
+  }
+  __device__ static uint32_t pair(const uint32_t* w, int p, uint32_t, uint32_t) { return w[p]; }
+};
+
+// LDS: kStages steps of A, kGroups groups of four blocks of W (bf16: a step's W
+// beside its A), and a place for the unused part of a group's last load.
+template <class F, int TM, int BR>
+struct WideLds {
+  static constexpr uint32_t kMax = 160 * 1024;
+  static constexpr uint32_t kA = 64 * TM * 128;
+  static constexpr uint32_t kB = BR * 16 * F::kChunks;
+  static constexpr uint32_t kPad = F::kBf16 ? 0 : 1024;
+  static constexpr int kGroups = F::kBf16 ? 0 : 3 * kA + 3 * kB + kPad <= kMax ? 3 : 2;
+  static constexpr int kFit = (kMax - kPad - kGroups * kB) / (kA + (F::kBf16 ? kB : 0));
+  static constexpr int kStages = kFit < 5 ? kFit : 5;
+  static constexpr int kBStages = F::kBf16 ? kStages : kGroups;
+  static constexpr uint32_t kBytes = kStages * kA + kBStages * kB + kPad;
+};
+
+template <class F, int TM, int NMAT, int BR>
+__device__ __forceinline__ void wide_tile(const _Float16* __restrict__ Ax,
+                                          const float* __restrict__ rs,
+                                          const uint8_t* __restrict__ W0,
+                                          const uint8_t* __restrict__ W1, float* __restrict__ C,
+                                          uint32_t T, uint32_t N, uint32_t K) {
+  using L = WideLds<F, TM, BR>;
+  constexpr int NA = TM;  // A pieces per thread and step (64 TM rows x 8 / 512)
+  constexpr int NS = L::kStages;
+  constexpr int NG = L::kGroups;
+  constexpr uint32_t BN = BR / NMAT;          // columns of C
+  constexpr int WN = 4;                       // wavefronts in N (2 in M)
+  constexpr int MT = 2 * TM, NT = BR / 64;    // 16 x 16 blocks of a wavefront
+  extern __shared__ __attribute__((aligned(16))) uint8_t pf_wide[];
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) uint8_t*)pf_wide;
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // XCD-aware tile order, as the tile GEMM's: split, m, n with n fastest
+  const uint32_t gx = gridDim.x, gy = gridDim.y, gz = gridDim.z, G = gx * gy * gz;
+  uint32_t w = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
+  if (G % 8 == 0) w = (w % 8) * (G / 8) + w / 8;
+  const uint32_t tn = w % gx, tm = (w / gx) % gy, z = w / (gx * gy);
+  const uint32_t m0 = tm * 64 * TM, n0 = tn * BN;
+  const uint32_t nq = K / 128;
+  const uint32_t q_begin = (uint32_t)((uint64_t)nq * z / gz);
+  const uint32_t q_end = (uint32_t)((uint64_t)nq * (z + 1) / gz);
+  const uint32_t s_end = 4 * q_end;
+  const size_t row_bytes = F::kBf16 ? (size_t)K * 2 : (size_t)nq * (16 * F::kChunks);
+
+  // A: piece c = 512 i + tid of a step is row c / 8, position c % 8, and comes
+  // from chunk (c % 8) ^ swizzle(row); rows past T load row T - 1
+  auto swz = [](uint32_t r) { return (r & 7) ^ ((r >> 3) & 1); };
+  uint32_t a_off[NA];
+#pragma unroll
+  for (int i = 0; i < NA; i++) {
+    const uint32_t r = 64 * i + (tid >> 3);
+    a_off[i] = (min(m0 + r, T - 1) - m0) * (4 * K) + 16 * ((tid & 7) ^ swz(r));
+  }
+  const uint8_t* a_base = reinterpret_cast<const uint8_t*>(Ax) + (size_t)m0 * 4 * K;
+  auto load_a = [&](uint32_t step, uint32_t st) {
+    const uint8_t* base = a_base + (size_t)min(step, s_end - 1) * 128;
+#pragma unroll
+    for (int i = 0; i < NA; i++)
+      load_lds16(a_off[i], base, lds0 + st * L::kA + 8192 * i + 1024 * wave);
+  };
+  // W: piece c of four blocks is row c / kChunks, part c % kChunks (bf16: of a
+  // step, row c / 4, position c % 4 from chunk (c % 4) ^ swizzle)
+  constexpr int NB = F::kBf16 ? F::per(BR, 0) : (BR * F::kChunks + PF_WIDE_NT - 1) / PF_WIDE_NT;
+  auto bswz = [](uint32_t r) { return ((r >> 1) ^ (r >> 2)) & 3; };
+  const uint8_t* b_src[NB];
+#pragma unroll
+  for (int i = 0; i < NB; i++) {
+    const uint32_t c = min(512u * i + tid, (uint32_t)BR * F::kChunks - 1);
+    const uint32_t r = c / F::kChunks, part = c % F::kChunks;
+    const uint8_t* W = r / BN ? W1 : W0;
+    b_src[i] = W + (size_t)min(n0 + r % BN, N - 1) * row_bytes +
+               16 * (F::kBf16 ? part ^ bswz(r) : part);
+  }
+  constexpr uint32_t kB0 = NS * L::kA, kPad0 = kB0 + L::kBStages * L::kB;
+  auto load_b = [&](int i, uint32_t unit, uint32_t st) {  // unit: a group of four (bf16: a step)
+    const uint32_t step_bytes = F::kBf16 ? 64 : 16 * F::kChunks;
+    const uint32_t last = (F::kBf16 ? s_end : q_end) - 1;
+    // a group's last load may need fewer wavefronts: the others' goes to the pad
+    const bool pad = 512u * i + 64u * wave >= (uint32_t)BR * F::kChunks;
+    load_lds16(b_src[i] + (size_t)min(unit, last) * step_bytes,
+               lds0 + (pad ? kPad0 : kB0 + st * L::kB + 8192 * i + 1024 * wave));
+  };
+
+  const uint32_t wm = (wave / WN) * (16 * MT), wn = wave % WN, g = lane >> 4, l16 = lane & 15;
+  // this lane's bytes of an A row (hi halves: chunk g, lo: 4 + g) and its
+  // weight rows (a pair: the first half of the blocks gate, the others the
+  // same columns of up)
+  const uint32_t a_hi = (wm + l16) * 128 + 16 * (g ^ swz(l16));
+  const uint32_t a_lo = (wm + l16) * 128 + 16 * ((4 + g) ^ swz(l16));
+  auto b_row = [&](int c) -> uint32_t {
+    return NMAT == 2 ? BN * (c / (NT / 2)) + 8 * NT * wn + 16 * (c % (NT / 2)) + l16
+                     : 16 * NT * wn + 16 * c + l16;
+  };
+  auto read_raw = [&](uint32_t (&r)[NT][F::kRaw], float (&d)[NT], uint32_t bst, int j) {
+#pragma unroll
+    for (int c = 0; c < NT; c++) {
+      if constexpr (F::kBf16)
+        F::raw(pf_wide + kB0 + bst * L::kB + b_row(c) * 64 + 16 * (g ^ bswz(l16)), g, r[c], &d[c]);
+      else
+        F::raw(pf_wide + kB0 + bst * L::kB + b_row(c) * (16 * F::kChunks) + j * (4 * F::kChunks), g, r[c], &d[c]);
+    }
+  };
+  auto read_a = [&](half8 (&a)[2], uint32_t st, int i) {
+    a[0] = *reinterpret_cast<const half8*>(pf_wide + st * L::kA + a_hi + 2048 * i);
+    a[1] = *reinterpret_cast<const half8*>(pf_wide + st * L::kA + a_lo + 2048 * i);
+  };
+
+  f32x4 acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; i++)
+#pragma unroll
+    for (int c = 0; c < NT; c++) acc[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  uint32_t step = 4 * q_begin;
+  // first loads: the first groups of W and the first NS - 1 steps of A
+  constexpr int per_step = NA + (F::kBf16 ? NB : 0);
+#pragma unroll
+  for (int p = 0; p < NS - 1; p++) {
+    if constexpr (F::kBf16) {
+#pragma unroll
+      for (int i = 0; i < NB; i++) load_b(i, step + p, p);
+    } else if (p < NG - 1) {
+#pragma unroll
+      for (int i = 0; i < NB; i++) load_b(i, q_begin + p, p);
+    }
+    load_a(step + p, p);
+    if constexpr (!F::kBf16 && NS - 1 < NG - 1) {
+      if (p == NS - 2) {
+#pragma unroll
+        for (int i = 0; i < NB; i++) load_b(i, q_begin + p + 1, p + 1);
+      }
+    }
+  }
+  wait_loads_barrier<(NS - 2) * per_step>();
+  uint32_t st = 0, bq = 0;  // stages of this step's A and of this group's W
+  // the unpacking's constants, in registers (an instruction holds one literal)
+  uint32_t mask = 0x000F000Fu, magic = 0x64006400u;
+  if constexpr (F::kChunks == 9) magic = 0x64646464u;
+  asm("" : "+v"(mask), "+s"(magic));
+  half8 a[2][2];
+  uint32_t raw[NT][F::kRaw];
+  u32x4 b[NT], bn[NT];
+  float d[NT], dn[NT], dp[NT];  // this step's scales, the next one's, the previous one's
+  f32x4 t[2][NT];               // block sums of 16 rows: this one's, the previous one's
+#pragma unroll
+  for (int c = 0; c < NT; c++) {
+    dp[c] = 0.f;
+    t[1][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+  static_assert(MT % 2 == 0, "the last 16 rows' sums are in t[1]");
+  read_raw(raw, d, 0, 0);
+  read_a(a[0], 0, 0);
+#pragma unroll
+  for (int c = 0; c < NT; c++)
+#pragma unroll
+    for (int p = 0; p < 4; p++) b[c][p] = F::pair(raw[c], p, mask, magic);
+
+  for (uint32_t q = q_begin; q < q_end; q++) {
+    int nload = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      // loads of a later step's operands, into the stage that the previous
+      // step read (every wave has passed a barrier since)
+      uint32_t nst = st + NS - 1;
+      nst = nst >= (uint32_t)NS ? nst - NS : nst;
+      if constexpr (F::kBf16) {
+#pragma unroll
+        for (int i = 0; i < NB; i++) load_b(i, step + NS - 1, nst);
+      } else {
+        const uint32_t nbq = bq == 0 ? NG - 1 : bq - 1;
+#pragma unroll
+        for (int p = 0; p < F::per(BR, j); p++) load_b(nload + p, q + NG - 1, nbq);
+        nload += F::per(BR, j);
+      }
+      load_a(step + NS - 1, nst);
+      const uint32_t sn = st + 1 == (uint32_t)NS ? 0 : st + 1;
+      // quantized: the next step's words are in LDS already (of the next group
+      // since the barrier of this group's third step); they are unpacked
+      // between the MFMAs
+      if constexpr (!F::kBf16) read_raw(raw, dn, j < 3 ? bq : bq + 1 == (uint32_t)NG ? 0 : bq + 1, (j + 1) & 3);
+#pragma unroll
+      for (int i = 0; i < MT; i++) {
+        if (i == MT - 1) {
+          // The next step's operands have landed for every wave: of the loads
+          // issued since, those of the last NS - 2 steps may be in flight; with
+          // two groups of W, in a group's third step only the A of two steps
+          // (the next group's last W went out in the second, ahead of that A).
+          constexpr int flight = (NS - 2) * per_step;
+          if (!F::kBf16 && NG == 2 && j == 2)
+            wait_loads_barrier<flight < 2 * NA ? flight : 2 * NA>();
+          else
+            wait_loads_barrier<flight>();
+          if constexpr (F::kBf16) read_raw(raw, dn, sn, 0);
+          read_a(a[(i + 1) & 1], sn, 0);
+        } else {
+          read_a(a[(i + 1) & 1], st, i + 1);
+        }
+        // (the compiler would sink the reads to just ahead of their use)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+          for (int c = 0; c < NT; c++) {
+            if constexpr (F::kBf16) {
+              acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  __builtin_bit_cast(bf16x8, a[i & 1][h]), __builtin_bit_cast(bf16x8, b[c]), acc[i][c], 0, 0, 0);
+            } else {
+              // one MFMA, then two scale FMAs of the previous 16 rows and a
+              // share of the unpacking: an MFMA that finds the matrix pipe
+              // busy holds up the SIMD's vector instructions too
+              t[i & 1][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                  a[i & 1][h], __builtin_bit_cast(half8, b[c]), h ? t[i & 1][c] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+              const int slot = h * NT + c;
+#pragma unroll
+              for (int e = 2 * slot; e < 2 * slot + 2; e++)
+                acc[(i + MT - 1) % MT][e / 4][e % 4] += (i ? d : dp)[e / 4] * t[(i + 1) & 1][e / 4][e % 4];
+              if (i > 0) {
+                constexpr int slots = (MT - 1) * 2 * NT, pairs = 4 * NT;
+                const int u = (i - 1) * 2 * NT + slot;
+#pragma unroll
+                for (int p = u * pairs / slots; p < (u + 1) * pairs / slots; p++)
+                  bn[p / 4][p % 4] = F::pair(raw[p / 4], p % 4, mask, magic);
+              }
+            }
+          }
+      }
+#pragma unroll
+      for (int c = 0; c < NT; c++) {
+        if constexpr (F::kBf16) {
+#pragma unroll
+          for (int p = 0; p < 4; p++) b[c][p] = raw[c][p];
+        } else {
+          b[c] = bn[c];
+          dp[c] = d[c];
+          d[c] = dn[c];
+        }
+      }
+      step++;
+      st = sn;
+    }
+    bq = bq + 1 == (uint32_t)NG ? 0 : bq + 1;
+  }
+  if constexpr (!F::kBf16) {
+#pragma unroll
+    for (int e = 0; e < 4 * NT; e++) acc[MT - 1][e / 4][e % 4] += dp[e / 4] * t[1][e / 4][e % 4];
+  }
+  // no load to LDS may outlive the workgroup
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+
+  // epilogue: result register e of lane l -> row 4 (l / 16) + e, column l % 16
+#pragma unroll
+  for (int i = 0; i < MT; i++) {
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+      const uint32_t row = m0 + wm + 16 * i + 4 * g + e;
+      if (row >= T) continue;
+      const float sr = rs[row];
+      if constexpr (NMAT == 2) {
+#pragma unroll
+        for (int c = 0; c < NT / 2; c++) {
+          const uint32_t col = n0 + 8 * NT * wn + 16 * c + l16;
+          if (col >= N) continue;
+          const float x = acc[i][c][e] * sr, y = acc[i][c + NT / 2][e] * sr;
+          if (gz > 1) {
+            C[((size_t)(2 * z) * T + row) * N + col] = x;
+            C[((size_t)(2 * z + 1) * T + row) * N + col] = y;
+          } else {
+            C[(size_t)row * N + col] = gelu_tanh(x) * y;
+          }
+        }
+      } else {
+#pragma unroll
+        for (int c = 0; c < NT; c++) {
+          const uint32_t col = n0 + 16 * NT * wn + 16 * c + l16;
+          if (col < N) C[((size_t)z * T + row) * N + col] = acc[i][c][e] * sr;
+        }
+      }
+    }
+  }
+}
+
+// (two wavefronts per SIMD at least; the small tiles' registers and LDS let a
+// second workgroup onto a CU)
+#define GH_WIDE_TM(FMT, F, TM, BR)                                                            \
+  extern "C" __global__ __launch_bounds__(PF_WIDE_NT) __attribute__((amdgpu_waves_per_eu(2)))  \
+  void gh_pf_wgemm_##FMT##_m##TM##_n##BR##_k(const _Float16* Ax, const float* rs,              \
+                                             const uint8_t* W, float* C, uint32_t T,           \
+                                             uint32_t N, uint32_t K) {                         \
+    wide_tile<F, TM, 1, BR>(Ax, rs, W, W, C, T, N, K);                                         \
+  }                                                                                            \
+  extern "C" __global__ __launch_bounds__(PF_WIDE_NT) __attribute__((amdgpu_waves_per_eu(2)))  \
+  void gh_pf_wgateup_##FMT##_m##TM##_n##BR##_k(const _Float16* Ax, const float* rs,            \
+                                               const uint8_t* Wg, const uint8_t* Wu,           \
+                                               float* Act, uint32_t T, uint32_t N,             \
+                                               uint32_t K) {                                   \
+    wide_tile<F, TM, 2, BR>(Ax, rs, Wg, Wu, Act, T, N, K);                                     \
+  }
+#define GH_WIDE(FMT, F)                                                            \
+  GH_WIDE_TM(FMT, F, 1, 256) GH_WIDE_TM(FMT, F, 2, 256) GH_WIDE_TM(FMT, F, 3, 256) \
+  GH_WIDE_TM(FMT, F, 4, 256) GH_WIDE_TM(FMT, F, 1, 128) GH_WIDE_TM(FMT, F, 2, 128) \
+  GH_WIDE_TM(FMT, F, 3, 128)
+GH_WIDE(q4, WQ4)
+GH_WIDE(q8, WQ8)
+GH_WIDE(bf16, WBf16)
+
 // The row scale of the GEMM's A operand for a row whose largest |x| is m:
 // s = 2^(e - 14) with 2^(e-1) <= m < 2^e (1 for m = 0), so every |x| / s
 // < 2^14 fits fp16; returns s and sets *inv = 1 / s (both exact).
@@ -593,7 +1001,6 @@ extern "C" __global__ __launch_bounds__(PF_NT) void gh_pf_splitk_k(const float* 
 // threads per token); plane z then carries that scale instead of the row's.
 // This saves the separate split launch (gh_pf_halves_k).
 // ---------------------------------------------------------------------------
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 struct SQ4 {  // Q4_0 (src/quant.zig:55-90): {f32 d, 4 words of nibbles}
   static constexpr uint32_t kBlockBytes = 20;

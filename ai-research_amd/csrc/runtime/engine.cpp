@@ -1,6 +1,7 @@
 // engine.cpp -- kernel-level entry points, the counterpart of GpuEngine's
 // record* helpers (src/gpu/kernels.zig:80-142): shape checks, launch-shape
 // selection, and the launch on the context stream.
+#include <math.h>
 #include <stdlib.h>
 #include <string.h>
 
@@ -487,6 +488,111 @@ bool stream_ok(const gh_context* ctx, gh_quant_mode mode, uint32_t T, uint32_t K
          stream_kr(ctx, mode, W1 != nullptr, T, K / 32) != 0 &&
          getenv("GH_PF_NO_STREAM") == nullptr;
 }
+
+// ---- the wide tile GEMM (gh_pf_wgemm_* / gh_pf_wgateup_*) ----
+// A workgroup's tile: 64 tm tokens by br weight rows (a gate/up pair: br / 2 of
+// each matrix), K in nz splits.
+struct WideShape {
+  uint32_t tm = 0, br = 256, nz = 1;
+};
+
+// LDS bytes of a tile (WideLds in prefill.hip)
+unsigned wide_lds(gh_quant_mode mode, uint32_t tm, uint32_t br) {
+  const unsigned max = 160 * 1024, a = 64 * tm * 128;
+  const unsigned b = br * 16 * (mode == GH_QUANT_Q4 ? 5 : mode == GH_QUANT_Q8 ? 9 : 4);
+  if (mode == GH_QUANT_NONE) return std::min(5u, max / (a + b)) * (a + b);
+  const unsigned pad = 1024, groups = 3 * a + 3 * b + pad <= max ? 3 : 2;
+  return std::min(5u, (max - pad - groups * b) / a) * a + groups * b + pad;
+}
+
+// The cheapest tile and split by a cost in us: rounds of workgroups over the
+// CUs (the 64 x 128 tile fits a CU twice) times steps of one block, plus the
+// split planes' traffic.  The constants are fitted to 297 measured products
+// (three weight modes, 9 shapes of 2048 - 15360 rows by 1536 - 15360, 11
+// lengths of 49 - 512 tokens, up to 30 tiles and splits each): the tile taken
+// is 1.0% behind the best one in the mean and 14% at worst, and ahead of the
+// 64- and 128-row tiles of one K block per barrier in every one of them
+// (1.02 to 1.75x).  GH_PF_WIDE="tm,nz,br" forces one.
+WideShape wide_shape(const gh_context* ctx, bool pair, uint32_t T, uint32_t N, uint32_t K) {
+  const uint32_t cus = (uint32_t)ctx->num_cus, nq = K / 128;
+  WideShape best;
+  if (const char* env = getenv("GH_PF_WIDE")) {
+    unsigned t = 0, z = 0, r = 0;
+    if (sscanf(env, "%u,%u,%u", &t, &z, &r) == 3 && t >= 1 && z >= 1 &&
+        ((r == 256 && t <= 4) || (r == 128 && t <= 3)))
+      return WideShape{t, r, std::min(std::min(z, nq), 64u)};
+  }
+  static const double step_us[2][4] = {{0.37, 0.55, 0.79, 0}, {0.75, 1.04, 1.27, 1.63}};
+  double least = 0;
+  for (uint32_t br = 128; br <= 256; br += 128) {
+    for (uint32_t tm = 1; tm <= (br == 128 ? 3u : 4u); tm++) {
+      const uint32_t bn = pair ? br / 2 : br, rows = 64 * tm;
+      const uint64_t tiles = (uint64_t)((N + bn - 1) / bn) * ((T + rows - 1) / rows);
+      const bool twice = br == 128 && tm == 1;
+      const uint32_t zmax = (uint32_t)std::min<uint64_t>(std::min(nq, 64u), 2 * cus / tiles);
+      for (uint32_t nz = 1; nz <= std::max(1u, zmax); nz++) {
+        const double load = (double)(tiles * nz) / cus;
+        const double rounds = load <= 1 ? 1 : twice ? ceil(2 * load) / 2 : ceil(load);
+        double cost = rounds * (4.0 * ((nq + nz - 1) / nz) * step_us[br / 256][tm - 1] + 19);
+        if (nz > 1) cost += 1.5 + 1.03 * nz * (pair ? 2 : 1) * T * (double)N * 8 / 4e6;
+        if (best.tm == 0 || cost < least) {
+          least = cost;
+          best = WideShape{tm, br, nz};
+        }
+      }
+    }
+  }
+  return best;
+}
+
+// Every operand piece is 16 bytes: K a multiple of 128 (four quant blocks),
+// W 16-byte aligned.  Other products, and a forced split count of the tile
+// GEMM (GH_PF_SPLIT), take that one.
+bool wide_ok(uint32_t K, const void* W0, const void* W1) {
+  return K % 128 == 0 &&
+         !((reinterpret_cast<uintptr_t>(W0) | reinterpret_cast<uintptr_t>(W1 ? W1 : W0)) & 15) &&
+         getenv("GH_PF_NO_WIDE") == nullptr && getenv("GH_PF_SPLIT") == nullptr;
+}
+
+gh_status launch_prefill_wide(gh_context* ctx, gh_quant_mode mode, const void* W0, const void* W1,
+                              const void* Ax, const float* rs, float* C, uint32_t T, uint32_t N,
+                              uint32_t K, const float** planes, uint32_t* nplanes) {
+  const bool pair = W1 != nullptr;
+  const WideShape sh = wide_shape(ctx, pair, T, N, K);
+  const uint32_t bn = pair ? sh.br / 2 : sh.br, nmat = pair ? 2u : 1u;
+  uint32_t nz = sh.nz;
+  float* out = C;
+  if (nz > 1) {
+    const size_t need = (size_t)nz * nmat * T * N * sizeof(float);
+    gh_status st = ctx->ensure_zeroed(&ctx->gemm_scratch, &ctx->gemm_scratch_bytes, need);
+    if (st != GH_OK) return st;
+    out = static_cast<float*>(ctx->gemm_scratch);
+  }
+  const std::string name = std::string(pair ? "gh_pf_wgateup_" : "gh_pf_wgemm_") +
+                           (mode == GH_QUANT_Q8 ? "q8" : mode == GH_QUANT_NONE ? "bf16" : "q4") +
+                           "_m" + std::to_string(sh.tm) + "_n" + std::to_string(sh.br) + "_k";
+  const dim3 grid((N + bn - 1) / bn, (T + 64 * sh.tm - 1) / (64 * sh.tm), nz);
+  const unsigned lds = wide_lds(mode, sh.tm, sh.br);
+  gh_status st;
+  if (pair) {
+    void* args[] = {const_cast<void**>(&Ax), const_cast<float**>(&rs), const_cast<void**>(&W0),
+                    const_cast<void**>(&W1), &out, &T, &N, &K};
+    st = ctx->launch(name, grid, dim3(512), lds, args);
+  } else {
+    void* args[] = {const_cast<void**>(&Ax), const_cast<float**>(&rs), const_cast<void**>(&W0),
+                    &out, &T, &N, &K};
+    st = ctx->launch(name, grid, dim3(512), lds, args);
+  }
+  if (planes) {
+    *planes = nz > 1 ? out : C;
+    *nplanes = nz;
+  }
+  if (st != GH_OK || nz == 1 || planes) return st;
+  const uint64_t tn = (uint64_t)T * N;
+  const unsigned rgrid = (unsigned)std::min<uint64_t>((tn + 255) / 256, 4ull * ctx->num_cus);
+  void* rargs[] = {&out, &C, &T, &N, &nz, const_cast<uint32_t*>(&nmat)};
+  return ctx->launch("gh_pf_splitk_k", dim3(rgrid), dim3(256), 0, rargs);
+}
 }  // namespace
 
 gh_status launch_prefill_gemm_split(gh_context* ctx, gh_quant_mode mode, const void* W0,
@@ -509,6 +615,11 @@ gh_status launch_prefill_gemm_split(gh_context* ctx, gh_quant_mode mode, const v
   if (pair && planes) return fail(GH_ERR_INVALID, "prefill GEMM: unsummed planes of a gate/up pair");
   if (stream_ok(ctx, mode, T, K, W0, W1))
     return launch_prefill_stream(ctx, mode, W0, W1, Ax, rs, C, T, N, K, planes, nplanes, false);
+  // Longer batches take the wide tile, 1.02-1.75x the speed of the tiles below
+  // wherever both were measured (wide_shape).  Those stay for K that is no
+  // multiple of 128 and for weights that are not 16-byte aligned.
+  if (wide_ok(K, W0, W1))
+    return launch_prefill_wide(ctx, mode, W0, W1, Ax, rs, C, T, N, K, planes, nplanes);
   // A product without planes of 256k + 1..127 tokens (a 288-token gate+up:
   // 720 tiles, the last 240 three-quarters padding) runs as two products: the
   // multiple of 256 on the tiles, the rest as its own product (the

@@ -89,6 +89,56 @@ def test_prefill_gate_up_large_tiles(gpu, mode, T, N, K):
         assert_close(got[t], ref[t], what="prefill GeGLU row %d" % t)
 
 
+# The wide tile GEMM (64 tm tokens by br weight rows, K in groups of four quant
+# blocks, split nz ways): each tile forced ("tm,nz,br") at the edges of its
+# range: one token past and short of a tile, ragged N on either side of a tile,
+# K of one group (every prefetch clamped), of two and of five (an uneven split),
+# more splits than groups.  "tile": the same products on the 64- and 128-row
+# tiles (GH_PF_NO_WIDE), which K = 160 and 1056 (no multiple of 128) and weights
+# off 16 bytes take by themselves.  The activations enter at 22 bits (bf16
+# weights: 16), so the fp64 product is met to a few 2^-22 (2^-16) of the row's
+# rms; the elementwise floor is a tenth of that rms, which leaves 2e-5 (1e-3).
+WIDE_SHAPES = [(49, 130, 128, "1,1,128"), (65, 257, 640, "1,2,128"), (64, 127, 256, "1,1,256"),
+               (129, 300, 640, "2,1,128"), (127, 513, 256, "2,4,256"), (128, 256, 128, "2,1,256"),
+               (193, 255, 384, "3,2,128"), (191, 700, 640, "3,3,256"), (257, 260, 640, "4,1,256"),
+               (255, 1000, 256, "4,2,256"), (512, 512, 384, "4,9,256"), (77, 1100, 1152, None),
+               (333, 390, 3840, None), (70, 200, 160, None), (150, 260, 1056, None),
+               (65, 257, 640, "tile"), (300, 128, 1024, "tile"), (130, 300, 640, "tile")]
+
+
+@pytest.mark.parametrize("mode", [gh.QUANT_Q4, gh.QUANT_Q8, gh.QUANT_NONE])
+@pytest.mark.parametrize("T,N,K,force", WIDE_SHAPES)
+def test_prefill_wide_tiles(gpu, monkeypatch, mode, T, N, K, force):
+    if force == "tile":
+        monkeypatch.setenv("GH_PF_NO_WIDE", "1")
+    elif force:
+        monkeypatch.setenv("GH_PF_WIDE", force)
+    rtol = 1e-3 if mode == gh.QUANT_NONE else 2e-5
+    gq, gdeq = quantized(N, K, mode, 390)
+    uq, udeq = quantized(N, K, mode, 391)
+    a = gh.synth_normal(T * K, 1, 392, 0.0, 1.0).reshape(T, K)
+    a64 = np.asarray(a, np.float64)
+    # guard rows behind the output: nothing is written past row T - 1
+    A, C = gpu.upload(a), gpu.alloc((T + 64) * N * 4)
+    gpu.fill_u32(C, 0x7FC12345, (T + 64) * N)
+
+    def result(what, ref):
+        out = C.read(np.uint32, (T + 64) * N).reshape(T + 64, N)
+        assert np.all(out[T:] == 0x7FC12345), what
+        assert_close(out[:T].view(np.float32), ref, rtol=rtol, what=what)
+
+    W, Wu = gpu.upload(gq), gpu.upload(uq)
+    gpu.prefill_gemm(mode, W, A, C, T, N, K)
+    result("wide GEMM", a64 @ gdeq.T)
+    gpu.prefill_gate_up_geglu(mode, W, Wu, A, C, T, N, K)
+    result("wide GeGLU", nr.gelu64(a64 @ gdeq.T) * (a64 @ udeq.T))
+    if mode != gh.QUANT_NONE and force is None:  # 4-byte aligned weights: the tiles
+        off = gpu.alloc(gq.nbytes + 4)
+        off.write(gq, 4)
+        gpu.prefill_gemm(mode, off.ptr + 4, A, C, T, N, K)
+        result("tile GEMM, 4-byte aligned weights", a64 @ gdeq.T)
+
+
 def test_prefill_gemm_row_range(gpu):
     # rows far outside fp16 range (1e6, 1e-7), a zero row and mixed magnitudes
     # within a row: the per-row power-of-two scale keeps every row exact to
