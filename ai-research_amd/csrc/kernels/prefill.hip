@@ -479,6 +479,15 @@ __device__ __forceinline__ void wait_loads_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
 }
 
+// The unpacking's constants, held in registers (an instruction takes one
+// literal at most).
+struct Unpack {
+  uint32_t lo = 0x000F000Fu, hi = 0x00F000F0u, magic, sixteenth = 0x2C002C00u, bias = 0xD480D480u;
+  __device__ explicit Unpack(bool q8) : magic(q8 ? 0x64646464u : 0x64006400u) {
+    asm("" : "+v"(lo), "+v"(hi), "+s"(magic), "+v"(sixteenth), "+s"(bias));
+  }
+};
+
 // A weight format of the wide tile.  Quantized: kChunks 16-byte pieces of a
 // row hold four blocks, and per(rows, j) pieces per thread of a group of four
 // blocks are loaded in step j of the four.  bf16: a step's 64 bytes of a row (4 pieces, swizzled), two per thread.
@@ -493,12 +502,21 @@ struct WQ4 {
     *d = __uint_as_float(p[0]);
     w[0] = p[1 + g];
   }
-  // the operand's pair p, as Q4W::ints (mask and magic: see wide_tile)
-  __device__ static uint32_t pair(const uint32_t* w, int p, uint32_t mask, uint32_t magic) {
+  // The operand's pair p, elements p and p + 4 of the word, as n - 8 exactly:
+  // nibbles under the exponent of 1024 are 1024 + n in the low position and
+  // 1024 + 16 n in the next, and one packed add of -1032, or a multiply-add by
+  // 1/16 and -72, leaves n - 8.  So only the upper half of the word is shifted.
+  __device__ static uint32_t pair(const uint32_t* w, int p, const Unpack& c) {
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
     uint32_t pr;
-    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(pr) : "v"(w[0] >> (4 * p)), "v"(mask), "s"(magic));
-    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, pr) + h2{(_Float16)-1032.0f, (_Float16)-1032.0f});
+    asm("v_and_or_b32 %0, %1, %2, %3" : "=v"(pr) : "v"(p < 2 ? w[0] : w[0] >> 8), "v"(p % 2 ? c.hi : c.lo), "s"(c.magic));
+    const h2 v = __builtin_bit_cast(h2, pr);
+    h2 o;
+    if (p % 2 == 0)
+      o = v + h2{(_Float16)-1032.0f, (_Float16)-1032.0f};
+    else
+      asm("v_pk_fma_f16 %0, %1, %2, %3" : "=v"(o) : "v"(v), "v"(c.sixteenth), "s"(c.bias));
+    return __builtin_bit_cast(uint32_t, o);
   }
 };
 struct WQ8 {
@@ -513,9 +531,9 @@ struct WQ8 {
   }
   // byte q + 128 under the exponent of 1024 is 1024 + (q + 128), exactly; the
   // packed add of -1152 leaves q
-  __device__ static uint32_t pair(const uint32_t* w, int p, uint32_t, uint32_t magic) {
+  __device__ static uint32_t pair(const uint32_t* w, int p, const Unpack& c) {
     typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    const uint32_t u = __builtin_amdgcn_perm(magic, w[p / 2] ^ 0x80808080u, p % 2 ? 0x07030702u : 0x07010700u);
+    const uint32_t u = __builtin_amdgcn_perm(c.magic, w[p / 2] ^ 0x80808080u, p % 2 ? 0x07030702u : 0x07010700u);
     return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, u) + h2{(_Float16)-1152.0f, (_Float16)-1152.0f});
   }
 };
@@ -528,7 +546,7 @@ struct WBf16 {
 #pragma unroll
     for (int k = 0; k < 4; k++) w[k] = v[k];
   }
-  __device__ static uint32_t pair(const uint32_t* w, int p, uint32_t, uint32_t) { return w[p]; }
+  __device__ static uint32_t pair(const uint32_t* w, int p, const Unpack&) { return w[p]; }
 };
 
 // LDS: kStages steps of A, kGroups groups of four blocks of W (bf16: a step's W
@@ -666,10 +684,7 @@ __device__ __forceinline__ void wide_tile(const _Float16* __restrict__ Ax,
   }
   wait_loads_barrier<(NS - 2) * per_step>();
   uint32_t st = 0, bq = 0;  // stages of this step's A and of this group's W
-  // the unpacking's constants, in registers (an instruction holds one literal)
-  uint32_t mask = 0x000F000Fu, magic = 0x64006400u;
-  if constexpr (F::kChunks == 9) magic = 0x64646464u;
-  asm("" : "+v"(mask), "+s"(magic));
+  const Unpack uc(F::kChunks == 9);
   half8 a[2][2];
   uint32_t raw[NT][F::kRaw];
   u32x4 b[NT], bn[NT];
@@ -686,7 +701,7 @@ __device__ __forceinline__ void wide_tile(const _Float16* __restrict__ Ax,
 #pragma unroll
   for (int c = 0; c < NT; c++)
 #pragma unroll
-    for (int p = 0; p < 4; p++) b[c][p] = F::pair(raw[c], p, mask, magic);
+    for (int p = 0; p < 4; p++) b[c][p] = F::pair(raw[c], p, uc);
 
   for (uint32_t q = q_begin; q < q_end; q++) {
     int nload = 0;
@@ -752,7 +767,7 @@ __device__ __forceinline__ void wide_tile(const _Float16* __restrict__ Ax,
                 const int u = (i - 1) * 2 * NT + slot;
 #pragma unroll
                 for (int p = u * pairs / slots; p < (u + 1) * pairs / slots; p++)
-                  bn[p / 4][p % 4] = F::pair(raw[p / 4], p % 4, mask, magic);
+                  bn[p / 4][p % 4] = F::pair(raw[p / 4], p % 4, uc);
               }
             }
           }
@@ -953,12 +968,10 @@ extern "C" __global__ __launch_bounds__(PF_NT) void gh_pf_splitk_k(const float* 
 // ---------------------------------------------------------------------------
 // Short batches (at most 48 tokens): the weight-streaming GEMM.
 //
-// With a few tokens the tile GEMM above spends each K step on one barrier
-// and one load round trip for a tile that is mostly padding, and reads its
-// weights at 0.8-1.5 TB/s.  Here every wavefront streams its own weight rows,
-// one register set of 16 rows x SB quant blocks in flight while the previous
-// set feeds the matrix cores, and the tokens take the MFMA's other
-// dimension: v_mfma_f32_16x16x32_f16 (or _bf16) with A = 16 tokens x 32 K
+// With a few tokens a tile is mostly padding, so here every wavefront streams
+// its own weight rows, one register set of 16 rows x SB quant blocks in flight
+// while the previous set feeds the matrix cores, and the tokens take the MFMA's
+// other dimension: v_mfma_f32_16x16x32_f16 (or _bf16) with A = 16 tokens x 32 K
 // (the activation halves, as the tile GEMM reads them) and B = 32 K x 16
 // weight rows (one quant block of each row, exact integers), so one MFMA
 // pair (hi, lo) covers one block of 16 rows and the rows' block scales apply
@@ -976,324 +989,381 @@ extern "C" __global__ __launch_bounds__(PF_NT) void gh_pf_splitk_k(const float* 
 // blocks (16-byte loads) of row l % 16, piece l / 16, so each row's SB
 // blocks arrive as one contiguous run.  (Loading each lane's MFMA fragment
 // directly, one scale and one word per block from 16 rows 2400 bytes apart,
-// reads at about 1.3 TB/s against 5.4-6.0 TB/s for these runs.)  The wave
-// then writes the set to its
-// own LDS rows and reads the fragments back; LDS keeps a wave's operations in
-// order, so no barrier is involved.  Bank conflicts: each 16-lane phase of a
-// set write covers 16 rows (one piece), and the row strides (84, 148 and 132
-// dwords) are 4 x odd modulo the 64 banks, so those writes and the fragment
-// reads (16 rows, 4 lane groups) land on distinct banks.  (With lane l on
-// row l / 4 a phase held 4 rows x 4 pieces at bank 20 (row + piece); the
-// gate+up's conflict cycles fell by a quarter with this mapping, its time
-// did not move.)
+// reads at about 1.3 TB/s against 5.4-6.0 TB/s for these runs.)  Lane group k
+// then holds whole blocks PB k + i of its rows, where the fragments want word
+// 1 + g in group g: a 4 x 4 transpose between registers and lane groups, four
+// v_permlane swaps for four blocks, in registers (six more spread the four
+// scales).  Taking the set through LDS instead (written as loaded, read back
+// as fragments) cost a round trip per set and most of the LDS.
 //
-// Workgroup (x, z) of NW waves owns row groups [NW RGW x, NW RGW (x + 1)) of
-// 16 rows and K blocks [z KR, z KR + KR) (KR and K / 32 multiples of 4): it
-// stages that slice of the T <= 16 TG activation rows in LDS once, and wave
-// w then streams row groups w, w + NW, ... with no further barrier.
-// gridDim.z > 1: plane z of [Z][NMAT][T][N] takes the raw sums times the row
-// scale, as the tile GEMM's split form writes them; gridDim.z = 1: C takes
-// the epilogue.
+// Workgroup (x, z) of 8 waves (4 for narrow products) owns RGW row units of 16
+// per wave (of each matrix of a gate/up pair, one after the other) and K blocks
+// [z KR, z KR + KR) (KR and K / 32 multiples of 4): it stages that slice of the
+// T <= 16 TG activation rows in LDS once, and wave w then streams its units with
+// no further barrier.  gridDim.z > 1: plane z of [Z][NMAT][T][N] takes the raw
+// sums times the row scale, as the tile GEMM's split form writes them;
+// gridDim.z = 1: C takes the epilogue.
+//
+// What bounds it: at a few tokens the weights' bytes and the start (launch,
+// first loads, staging), from 16 tokens the vector work per block (unpacking,
+// scale FMAs) beside the MFMAs.  Timing-only copies, gate/up of 16 tokens
+// (73.7 MB, 13.4 us at 5.5 TB/s): 28 us with its plane sum, 17-18 without the
+// arithmetic, 24 without all loads but the first.  Against the form through
+// LDS, us with the plane sums (Q4, 3 / 16 / 32 tokens): gate/up 31 / 34 / 46 ->
+// 25 / 28 / 39, QKV 13.1 / 15.1 / 18.1 -> 10.7 / 12.2 / 16.1, o 10.0 / 11.4 /
+// 13.5 -> 8.1 / 9.5 / 12.4, down 22 / 23 / 30 -> 16.7 / 19.6 / 25.2; Q8 gate/up of 16
+// and 32 tokens 51 / 70 -> 38 / 48.
 //
 // AF (the o and down inputs, and the kernel-level f32 entry points): A comes
 // as f32 rows, and the staging splits each token's slice itself, with a
-// power-of-two scale of its own (row_scale of the slice's largest |a|, 16
-// threads per token); plane z then carries that scale instead of the row's.
-// This saves the separate split launch (gh_pf_halves_k).
+// power-of-two scale of its own (row_scale of the slice's largest |a|); plane z
+// then carries that scale instead of the row's.  This saves the separate split
+// launch (gh_pf_halves_k).
 // ---------------------------------------------------------------------------
+// Register r of lane group k <-> register k of lane group r.
+__device__ __forceinline__ void transpose4(uint32_t& w0, uint32_t& w1, uint32_t& w2, uint32_t& w3) {
+  const auto a = __builtin_amdgcn_permlane32_swap(w0, w2, false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(w1, w3, false, false);
+  const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+  const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+  w0 = c[0];
+  w1 = c[1];
+  w2 = d[0];
+  w3 = d[1];
+}
+// d[k] = v of lane group k
+__device__ __forceinline__ void spread4(uint32_t v, float (&d)[4]) {
+  const auto a = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  const auto b = __builtin_amdgcn_permlane16_swap(a[0], a[0], false, false);
+  const auto c = __builtin_amdgcn_permlane16_swap(a[1], a[1], false, false);
+  d[0] = __uint_as_float(b[0]);
+  d[1] = __uint_as_float(b[1]);
+  d[2] = __uint_as_float(c[0]);
+  d[3] = __uint_as_float(c[1]);
+}
 
+// A streamed format: kPB blocks per lane and set.  take: block i of every lane
+// group's piece as the fragments' words (w[k]: block kPB k + i) and scales;
+// half: the operand from a fragment's words.
 struct SQ4 {  // Q4_0 (src/quant.zig:55-90): {f32 d, 4 words of nibbles}
   static constexpr uint32_t kBlockBytes = 20;
-  static constexpr int kPB = 4;  // blocks per lane and set (80 bytes)
+  static constexpr int kPB = 4, kWords = 1;  // 80 bytes
   static constexpr bool kBf16 = false;
   static constexpr uint32_t kFmt = 1;  // pf_store_group format of the A halves
-  // the fragment of block kb from an LDS row: scale d, word 1 + g as the
-  // fp16 pairs (n_j - 8, n_{j+4} - 8), j = 0..3, as Q4W::ints unpacks it
-  __device__ static half8 frag(const uint8_t* row, uint32_t kb, uint32_t g, float* d) {
-    const uint32_t* p = reinterpret_cast<const uint32_t*>(row + kb * kBlockBytes);
-    *d = __uint_as_float(p[0]);
-    const uint32_t w = p[1 + g];
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    const h2 bias = {(_Float16)-1032.0f, (_Float16)-1032.0f};
+  __device__ static void take(const uint32_t* r, int i, uint32_t (&w)[4][kWords], float (&d)[4]) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) w[k][0] = r[5 * i + 1 + k];
+    transpose4(w[0][0], w[1][0], w[2][0], w[3][0]);
+    spread4(r[5 * i], d);
+  }
+  __device__ static half8 half(const uint32_t* w, const Unpack& c) {
     u32x4 o;
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      const uint32_t pr = ((w >> (4 * j)) & 0x000F000Fu) | 0x64006400u;
-      o[j] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, pr) + bias);
-    }
+    for (int p = 0; p < 4; p++) o[p] = WQ4::pair(w, p, c);
     return __builtin_bit_cast(half8, o);
   }
 };
 
 struct SQ8 {  // Q8_0 (src/quant.zig:20-51): {f32 d, 8 words of int8}
   static constexpr uint32_t kBlockBytes = 36;
-  static constexpr int kPB = 4;  // 144 bytes
+  static constexpr int kPB = 4, kWords = 2;  // 144 bytes
   static constexpr bool kBf16 = false;
   static constexpr uint32_t kFmt = 0;
-  __device__ static half8 frag(const uint8_t* row, uint32_t kb, uint32_t g, float* d) {
-    const uint32_t* p = reinterpret_cast<const uint32_t*>(row + kb * kBlockBytes);
-    *d = __uint_as_float(p[0]);
-    const uint32_t w[2] = {p[1 + 2 * g], p[2 + 2 * g]};
-    half8 o;  // q as fp16, in K order
+  __device__ static void take(const uint32_t* r, int i, uint32_t (&w)[4][kWords], float (&d)[4]) {
 #pragma unroll
-    for (int k = 0; k < 2; k++)
+    for (int h = 0; h < 2; h++) {
 #pragma unroll
-      for (int n = 0; n < 4; n++) o[4 * k + n] = (_Float16)(int)(int8_t)((w[k] >> (8 * n)) & 0xFFu);
-    return o;
+      for (int k = 0; k < 4; k++) w[k][h] = r[9 * i + 1 + 2 * k + h];
+      transpose4(w[0][h], w[1][h], w[2][h], w[3][h]);
+    }
+    spread4(r[9 * i], d);
+  }
+  __device__ static half8 half(const uint32_t* w, const Unpack& c) {
+    u32x4 o;
+#pragma unroll
+    for (int p = 0; p < 4; p++) o[p] = WQ8::pair(w, p, c);
+    return __builtin_bit_cast(half8, o);
   }
 };
 
 struct SBf16 {  // bf16 rows: 32-element segments of 64 bytes, no scale
   static constexpr uint32_t kBlockBytes = 64;
-  static constexpr int kPB = 2;  // 128 bytes
+  static constexpr int kPB = 2, kWords = 4;  // 128 bytes
   static constexpr bool kBf16 = true;
   static constexpr uint32_t kFmt = 2;
-  __device__ static half8 frag(const uint8_t* row, uint32_t kb, uint32_t g, float* d) {
-    *d = 1.f;
-    return *reinterpret_cast<const half8*>(row + kb * kBlockBytes + 16 * g);
+  __device__ static void take(const uint32_t* r, int i, uint32_t (&w)[4][kWords], float (&d)[4]) {
+#pragma unroll
+    for (int h = 0; h < 4; h++) {
+#pragma unroll
+      for (int k = 0; k < 4; k++) w[k][h] = r[16 * i + 4 * k + h];
+      transpose4(w[0][h], w[1][h], w[2][h], w[3][h]);
+      d[h] = 1.f;
+    }
+  }
+  __device__ static half8 half(const uint32_t* w, const Unpack&) {
+    return __builtin_bit_cast(half8, u32x4{w[0], w[1], w[2], w[3]});
   }
 };
 
-template <class F>
-struct SSet {
-  static constexpr int SB = 4 * F::kPB;                          // blocks per set
-  static constexpr int NV = F::kPB * (int)F::kBlockBytes / 16;   // 16-byte loads per lane
-  static constexpr uint32_t RS = SB * F::kBlockBytes + 16;       // LDS row stride (bytes)
-  static constexpr uint32_t kWaveBytes = 16 * RS;                // one matrix's set
+// 8-element groups a thread holds while it splits f32 rows, for TG groups of
+// 16 tokens: a K slice of kr blocks has 4 kr groups per token, over the
+// workgroup's threads per token (a power of two)
+template <int TG>
+struct StreamStage {
+  static constexpr int kPer = TG <= 2 ? 10 : 16;
+  // threads per token of a workgroup of `waves` waves
+  __device__ static uint32_t tpt(uint32_t waves) { return waves * (TG <= 1 ? 4 : TG == 2 ? 2 : 1); }
 };
 
-#define PF_SLICE_MAX 32  // quant blocks per K slice (the AF staging holds 8 groups per thread)
-
-// NW waves per workgroup (NW * 64 threads), TG groups of 16 tokens (T <= 16 TG).
-template <class F, int NMAT, bool AF, int NW, int TG>
+// TG groups of 16 tokens (T <= 16 TG); TG = 0: at most 8 tokens, whose hi and
+// lo halves are rows 0-7 and 8-15 of one MFMA.
+template <class F, int NMAT, bool AF, int TG>
 __device__ __forceinline__ void stream_gemm(const _Float16* __restrict__ Ax,
                                             const float* __restrict__ rs,
                                             const uint8_t* __restrict__ W0,
                                             const uint8_t* __restrict__ W1,
                                             float* __restrict__ C, uint32_t T, uint32_t N,
                                             uint32_t K, uint32_t KR, uint32_t RGW) {
-  using S = SSet<F>;
-  constexpr int SB = S::SB, NV = S::NV, PB = F::kPB;
-  constexpr uint32_t NT = 64 * NW;
+  constexpr int PB = F::kPB, SB = 4 * PB, NV = PB * (int)F::kBlockBytes / 16;
+  constexpr bool kPack = TG == 0;
+  constexpr int NG = kPack ? 1 : TG, NH = kPack ? 1 : 2;  // token groups, halves apart
   extern __shared__ __attribute__((aligned(16))) uint8_t pf_slice[];
-  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t nthr = blockDim.x, nw = nthr / 64;
   const uint32_t g = lane >> 4, li = lane & 15;
   const uint32_t nb = K / 32, z = blockIdx.z;
   const uint32_t b0 = z * KR, nk = min(nb - b0, KR);  // the host keeps b0 < nb, 4 | nk
   const uint32_t stride = KR * 128 + 16;              // bytes per staged token row
   const size_t row_bytes = (size_t)nb * F::kBlockBytes;
-  const uint32_t kchunks = (nk + SB - 1) / SB;  // sets per row group
-  const uint32_t nchunks = RGW * kchunks;
-  const uint32_t rg0 = blockIdx.x * NW * RGW + wave;  // row group j of this wave: rg0 + NW j
-  // this wave's set rows, after the T staged token rows
-  uint8_t* wl = pf_slice + T * stride + wave * NMAT * S::kWaveBytes;
+  const uint32_t kchunks = (nk + SB - 1) / SB;  // sets per row unit
+  const uint32_t nchunks = RGW * NMAT * kchunks;
+  const uint32_t u0 = blockIdx.x * nw * RGW + wave;  // unit j of this wave: u0 + nw j
   // token rows of this lane's A fragments (one per group of 16 tokens):
   // tokens past T read token T - 1 (their D rows are never stored)
-  const uint8_t* al_row[TG];
+  const uint8_t* al_row[NG];
 #pragma unroll
-  for (int h = 0; h < TG; h++) al_row[h] = pf_slice + min(16 * h + li, T - 1) * stride + 16 * g;
+  for (int h = 0; h < NG; h++)
+    al_row[h] = pf_slice + min(kPack ? li & 7 : 16 * h + li, T - 1) * stride + 16 * g + (kPack && li >= 8 ? 64 : 0);
 
-  // Set c: row group j = c / kchunks, blocks kb0 .. kb0 + SB - 1 of the
-  // slice.  Lane l loads blocks kb0 + PB (l / 16) .. + PB - 1 of row l % 16
-  // (a piece that starts past the slice loads its last piece instead; those
-  // blocks are skipped).
-  u32x4 ra[NMAT][NV], rb[NMAT][NV];
-  auto load = [&](uint32_t c, u32x4(&r)[NMAT][NV]) {
+  // Set c: pass j = c / kchunks over the slice (unit j / NMAT; of a gate/up pair
+  // the gate rows, then the up rows), blocks kb0 .. kb0 + SB - 1.  Lane l loads
+  // blocks kb0 + PB (l / 16) .. + PB - 1 of row l % 16 (a piece past the slice
+  // loads the last one instead and enters as zeros).
+  u32x4 ra[NV], rb[NV];
+  auto load = [&](uint32_t c, u32x4(&r)[NV]) {
     const uint32_t j = c / kchunks, kb0 = (c % kchunks) * SB;
-    uint32_t row = (rg0 + NW * j) * 16 + li;
-    row = row < N ? row : N - 1;
     const uint32_t kb = min(kb0 + PB * g, nk - PB);
-    const size_t off = (size_t)row * row_bytes + (size_t)(b0 + kb) * F::kBlockBytes;
+    const uint32_t row = min(16 * (u0 + nw * (j / NMAT)) + li, N - 1);
+    const uint8_t* src = (j % NMAT ? W1 : W0) + (size_t)row * row_bytes + (size_t)(b0 + kb) * F::kBlockBytes;
 #pragma unroll
-    for (int i = 0; i < NV; i++) r[0][i] = *(gvec_ptr)(W0 + off + 16 * i);
-    if constexpr (NMAT == 2) {
-#pragma unroll
-      for (int i = 0; i < NV; i++) r[1][i] = *(gvec_ptr)(W1 + off + 16 * i);
-    }
+    for (int v = 0; v < NV; v++) r[v] = *(gvec_ptr)(src + 16 * v);
   };
 
-  // the first set is in flight while the slice is staged
-  load(0, ra);
-  __shared__ float slice_scale[16 * TG];  // AF: each token's scale for this slice
+  // The slice's loads first, then the first sets' (loads return in order, and
+  // the activations come from L2): the staging below runs while those are in
+  // flight.  AF: tpt threads per token; thread `sub` takes 8-element groups
+  // sub, sub + tpt, ... of the slice (4 nk of them).  Else: 16-byte chunks
+  // tid, tid + nthr, ... of the T rows' 8 nk each.
+  __shared__ float slice_scale[16 * NG];  // AF: each token's scale for this slice
+  constexpr int PER = StreamStage<TG>::kPer;
+  const uint32_t tpt = StreamStage<TG>::tpt(nw);
+  const uint32_t ngr = nk * 4, at = tid / tpt, sub = tid % tpt, chunks = T * nk * 8;
+  float xv[AF ? PER : 1][8];
+  u32x4 cv[AF ? 1 : 2 * PER];
   if constexpr (AF) {
-    // 16 threads per token, NT / 16 tokens per pass; thread `sub` takes
-    // 8-element groups sub, sub + 16, ... of the slice (nk / 4 of them: nk
-    // is a multiple of 4)
-    constexpr uint32_t TPP = NT / 16, PASSES = (16 * TG + TPP - 1) / TPP;
-    const float* A = reinterpret_cast<const float*>(Ax);
-#pragma unroll 1
-    for (uint32_t pass = 0; pass < PASSES; pass++) {
-      const uint32_t t = (tid >> 4) + pass * TPP, sub = tid & 15, per = nk / 4;
-      const bool on = t < T;
-      const float* src = A + (size_t)min(t, T - 1) * K + (size_t)b0 * 32;
-      float xv[PF_SLICE_MAX / 4][8];
-      float m = 0.f;
+    const float* src = reinterpret_cast<const float*>(Ax) + (size_t)min(at, T - 1) * K + (size_t)b0 * 32;
 #pragma unroll
-      for (int i = 0; i < PF_SLICE_MAX / 4; i++) {
-        if ((uint32_t)i < per) {
-          const float4 a = *reinterpret_cast<const float4*>(src + 8 * (sub + 16 * i));
-          const float4 b = *reinterpret_cast<const float4*>(src + 8 * (sub + 16 * i) + 4);
-          xv[i][0] = a.x; xv[i][1] = a.y; xv[i][2] = a.z; xv[i][3] = a.w;
-          xv[i][4] = b.x; xv[i][5] = b.y; xv[i][6] = b.z; xv[i][7] = b.w;
-#pragma unroll
-          for (int k = 0; k < 8; k++) m = fmaxf(m, fabsf(xv[i][k]));
-        }
-      }
-#pragma unroll
-      for (int off = 8; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
-      float inv;
-      const float sc = row_scale(m, &inv);
-      if (on) {
-#pragma unroll
-        for (int i = 0; i < PF_SLICE_MAX / 4; i++) {
-          if ((uint32_t)i < per) {
-            const uint32_t gi = sub + 16 * i;  // group gi: block gi / 4, part gi % 4
-            float y[8];
-#pragma unroll
-            for (int k = 0; k < 8; k++) y[k] = xv[i][k] * inv;
-            pf_store_group(y, F::kFmt,
-                           reinterpret_cast<_Float16*>(pf_slice + t * stride + (gi >> 2) * 128 +
-                                                       (gi & 3) * 16));
-          }
-        }
-        if (sub == 0) slice_scale[t] = sc;
-      }
+    for (int i = 0; i < PER; i++) {
+      if (tpt * i >= ngr) continue;  // uniform
+      const uint32_t gi = min(sub + tpt * i, ngr - 1);
+      const float4 a = *reinterpret_cast<const float4*>(src + 8 * gi);
+      const float4 b = *reinterpret_cast<const float4*>(src + 8 * gi + 4);
+      xv[i][0] = a.x; xv[i][1] = a.y; xv[i][2] = a.z; xv[i][3] = a.w;
+      xv[i][4] = b.x; xv[i][5] = b.y; xv[i][6] = b.z; xv[i][7] = b.w;
     }
   } else {
-    const uint32_t per_row = nk * 8;  // 16-byte chunks of one token's slice
-    const uint32_t total = T * per_row;
-#pragma unroll 4
-    for (uint32_t c = tid; c < total; c += NT) {
-      const uint32_t t = c / per_row, q = c % per_row;
-      const u32x4 v = *reinterpret_cast<const u32x4*>(Ax + (size_t)t * 2 * K + (size_t)b0 * 64 + 8 * q);
-      *reinterpret_cast<u32x4*>(pf_slice + t * stride + 16 * q) = v;
+#pragma unroll
+    for (int i = 0; i < 2 * PER; i++) {
+      if (nthr * i >= chunks) continue;  // uniform
+      const uint32_t c = min(tid + nthr * i, chunks - 1), t = c / (nk * 8), q = c % (nk * 8);
+      cv[i] = *reinterpret_cast<const u32x4*>(Ax + (size_t)t * 2 * K + (size_t)b0 * 64 + 8 * q);
+    }
+  }
+  asm volatile("" ::: "memory");
+  load(0, ra);
+  if (nchunks > 1) load(1, rb);
+  asm volatile("" ::: "memory");
+  if constexpr (AF) {
+    float m = 0.f;
+#pragma unroll
+    for (int i = 0; i < PER; i++) {
+      if (tpt * i >= ngr) continue;
+#pragma unroll
+      for (int k = 0; k < 8; k++) m = fmaxf(m, fabsf(xv[i][k]));
+    }
+    for (uint32_t off = tpt / 2; off > 0; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, 64));
+    float inv;
+    const float sc = row_scale(m, &inv);
+    if (at < T) {
+#pragma unroll
+      for (int i = 0; i < PER; i++) {
+        const uint32_t gi = sub + tpt * i;  // group gi: block gi / 4, part gi % 4
+        if (gi < ngr) {
+          float y[8];
+#pragma unroll
+          for (int k = 0; k < 8; k++) y[k] = xv[i][k] * inv;
+          pf_store_group(y, F::kFmt,
+                         reinterpret_cast<_Float16*>(pf_slice + at * stride + (gi >> 2) * 128 + (gi & 3) * 16));
+        }
+      }
+      if (sub == 0) slice_scale[at] = sc;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < 2 * PER; i++) {
+      const uint32_t c = tid + nthr * i;
+      if (c < chunks) *reinterpret_cast<u32x4*>(pf_slice + c / (nk * 8) * stride + 16 * (c % (nk * 8))) = cv[i];
     }
   }
   __syncthreads();
 
-  f32x4 acc[NMAT][TG];
+  const Unpack uc(F::kBlockBytes == 36);
+  f32x4 acc[NG], gate[NG];  // gate: the unit's sums of the first matrix of a pair
 #pragma unroll
-  for (int q = 0; q < NMAT; q++)
-#pragma unroll
-    for (int h = 0; h < TG; h++) acc[q][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int h = 0; h < NG; h++) acc[h] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+  // the sums of pass j to its unit's plane (or C), or kept; and clear them
   auto epilogue = [&](uint32_t j) {
-    const uint32_t n = (rg0 + NW * j) * 16 + li;
-    if (n >= N) return;
+    const bool keep = NMAT == 2 && j % 2 == 0;
+    const uint32_t n = 16 * (u0 + nw * (j / NMAT)) + li;
 #pragma unroll
-    for (int h = 0; h < TG; h++)
+    for (int h = 0; h < NG; h++) {
+      const f32x4 sum = acc[h];
+      acc[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (keep) {
+        gate[h] = sum;
+        continue;
+      }
 #pragma unroll
       for (int r = 0; r < 4; r++) {
-        const uint32_t t = 16 * h + 4 * g + r;
-        if (t >= T) continue;
-        const float sr = AF ? slice_scale[t] : rs[t];
-        if (gridDim.z > 1) {
+        float v[NMAT];
+        v[NMAT - 1] = sum[r];
+        if constexpr (NMAT == 2) v[0] = gate[h][r];
+        if constexpr (kPack) {  // rows 8 apart: lane groups 2 apart
 #pragma unroll
-          for (int q = 0; q < NMAT; q++)
-            C[((size_t)(z * NMAT + q) * T + t) * N + n] = acc[q][h][r] * sr;
-        } else if constexpr (NMAT == 1) {
-          C[(size_t)t * N + n] = acc[0][h][r] * sr;
-        } else {
-          C[(size_t)t * N + n] = gelu_tanh(acc[0][h][r] * sr) * (acc[1][h][r] * sr);
-        }
-      }
-  };
-
-  auto compute = [&](uint32_t c, const u32x4(&r)[NMAT][NV]) {
-    const uint32_t j = c / kchunks, kb0 = (c % kchunks) * SB;
-    // the set into this wave's LDS rows: lane l's piece l / 16 of row l % 16
-#pragma unroll
-    for (int q = 0; q < NMAT; q++)
-#pragma unroll
-      for (int i = 0; i < NV; i++)
-        *reinterpret_cast<u32x4*>(wl + q * S::kWaveBytes + li * S::RS + g * PB * F::kBlockBytes +
-                                  16 * i) = r[q][i];
-#pragma unroll
-    for (int u = 0; u < SB; u++) {
-      const uint32_t kb = kb0 + u;
-      if (kb < nk) {  // uniform over the wave
-        half8 ah[TG], al[TG];
-#pragma unroll
-        for (int h = 0; h < TG; h++) {
-          ah[h] = *reinterpret_cast<const half8*>(al_row[h] + kb * 128);
-          al[h] = *reinterpret_cast<const half8*>(al_row[h] + kb * 128 + 64);
-        }
-#pragma unroll
-        for (int q = 0; q < NMAT; q++) {
-          float d;
-          const half8 b = F::frag(wl + q * S::kWaveBytes + li * S::RS, (uint32_t)u, g, &d);
-#pragma unroll
-          for (int h = 0; h < TG; h++) {
-            if constexpr (F::kBf16) {
-              f32x4 t = acc[q][h];
-              t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, ah[h]),
-                                                          __builtin_bit_cast(bf16x8, b), t, 0, 0, 0);
-              t = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, al[h]),
-                                                          __builtin_bit_cast(bf16x8, b), t, 0, 0, 0);
-              acc[q][h] = t;
-            } else {
-              f32x4 blk = {0.f, 0.f, 0.f, 0.f};
-              blk = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[h], b, blk, 0, 0, 0);
-              blk = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[h], b, blk, 0, 0, 0);
-#pragma unroll
-              for (int e = 0; e < 4; e++) acc[q][h][e] += d * blk[e];
-            }
+          for (int q = 0; q < NMAT; q++) {
+            const auto o = __builtin_amdgcn_permlane32_swap(__float_as_uint(v[q]), __float_as_uint(v[q]), false, false);
+            v[q] = __uint_as_float(o[0]) + __uint_as_float(o[1]);
           }
+        }
+        const uint32_t t = 16 * h + 4 * g + r;
+        if (t >= T || n >= N) continue;
+        const float sr = AF ? slice_scale[t] : rs[t];
+        if (NMAT == 2 && gridDim.z == 1) {
+          C[(size_t)t * N + n] = gelu_tanh(v[0] * sr) * (v[NMAT - 1] * sr);
+        } else {
+#pragma unroll
+          for (int q = 0; q < NMAT; q++) C[((size_t)(NMAT * z + q) * T + t) * N + n] = v[q] * sr;
         }
       }
     }
-    if (c % kchunks == kchunks - 1) {  // the row group's last set
-      epilogue(j);
+  };
+
+  // set c into the sums
+  auto compute = [&](uint32_t c, u32x4(&r)[NV]) {
+    const uint32_t kb0 = (c % kchunks) * SB;
+    if (kb0 + SB > nk) {  // the slice's last set is partial
+      if (kb0 + PB * g >= nk) {
 #pragma unroll
-      for (int q = 0; q < NMAT; q++)
+        for (int i = 0; i < NV; i++) r[i] = u32x4{0, 0, 0, 0};
+      }
+    }
+    // Blocks PB k + i in the order i, then k.  While a block's MFMAs run, the
+    // next one's activations are on their way from LDS and its weights are
+    // unpacked; its scale FMAs follow.
+    uint32_t flat[4 * NV];
 #pragma unroll
-        for (int h = 0; h < TG; h++) acc[q][h] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int e = 0; e < 4 * NV; e++) flat[e] = r[e / 4][e % 4];
+    auto read_a = [&](half8(&x)[NH][NG], int p) {
+      const uint32_t kb = min(kb0 + PB * (p % 4) + p / 4, nk - 1);
+#pragma unroll
+      for (int h = 0; h < NG; h++)
+#pragma unroll
+        for (int s = 0; s < NH; s++)
+          x[s][h] = *reinterpret_cast<const half8*>(al_row[h] + kb * 128 + 64 * s);
+    };
+    half8 x[2][NH][NG], b;
+    uint32_t w[4][F::kWords];
+    float d[2][4];
+    read_a(x[0], 0);
+    F::take(flat, 0, w, d[0]);
+    b = F::half(w[0], uc);
+#pragma unroll
+    for (int p = 0; p < SB; p++) {
+      if (p + 1 < SB) read_a(x[(p + 1) & 1], p + 1);
+      // (the compiler would sink the reads to just ahead of their use)
+      __builtin_amdgcn_sched_barrier(0);
+      f32x4 t[NG];
+#pragma unroll
+      for (int s = 0; s < NH; s++)
+#pragma unroll
+        for (int h = 0; h < NG; h++) {
+          const half8 v = x[p & 1][s][h];
+          if constexpr (F::kBf16)
+            acc[h] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, v),
+                                                             __builtin_bit_cast(bf16x8, b), acc[h], 0, 0, 0);
+          else
+            t[h] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v, b, s ? t[h] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+        }
+      if (p + 1 < SB) {
+        if (p % 4 == 3) F::take(flat, p / 4 + 1, w, d[(p / 4 + 1) & 1]);
+        b = F::half(w[(p + 1) % 4], uc);
+      }
+      if constexpr (!F::kBf16) {
+#pragma unroll
+        for (int h = 0; h < NG; h++) {
+#pragma unroll
+          for (int e = 0; e < 4; e++) acc[h][e] += d[(p / 4) & 1][p % 4] * t[h][e];
+          // (pinned here: put off, the FMAs keep every block's sums in registers)
+          asm volatile("" : "+v"(acc[h]));
+        }
+      }
     }
   };
 
   for (uint32_t c = 0; c < nchunks; c += 2) {
-    if (c + 1 < nchunks) load(c + 1, rb);
     compute(c, ra);
+    if (c % kchunks == kchunks - 1) epilogue(c / kchunks);
+    if (c + 2 < nchunks) load(c + 2, ra);
     if (c + 1 < nchunks) {
-      if (c + 2 < nchunks) load(c + 2, ra);
       compute(c + 1, rb);
+      if ((c + 1) % kchunks == kchunks - 1) epilogue((c + 1) / kchunks);
+      if (c + 3 < nchunks) load(c + 3, rb);
     }
   }
 }
 
-// 4-wave workgroups for up to 16 tokens; 8-wave workgroups for 17-32 tokens
-// (two token groups per wave sharing each weight fragment; the 32 staged
-// token rows serve 8 waves' row groups, which keeps 16-block slices in LDS)
-// and for 33-48 tokens (three groups per wave, narrower slices where LDS
-// needs them).
-#define GH_SGEMM(NAME, F, NMAT, AF)                                                          \
-  extern "C" __global__ __launch_bounds__(256) void NAME##_k(                               \
+// t0: up to 8 tokens, t1 - t3: up to 16, 32, 48
+#define GH_SGEMM_TG(NAME, F, NMAT, AF, TG)                                                   \
+  extern "C" __global__ __launch_bounds__(512) void NAME##_t##TG##_k(                       \
       const _Float16* Ax, const float* rs, const uint8_t* W0, const uint8_t* W1, float* C,  \
       uint32_t T, uint32_t N, uint32_t K, uint32_t KR, uint32_t RGW) {                      \
-    stream_gemm<F, NMAT, AF, 4, 1>(Ax, rs, W0, W1, C, T, N, K, KR, RGW);                    \
-  }                                                                                         \
-  extern "C" __global__ __launch_bounds__(512) void NAME##_t2_k(                            \
-      const _Float16* Ax, const float* rs, const uint8_t* W0, const uint8_t* W1, float* C,  \
-      uint32_t T, uint32_t N, uint32_t K, uint32_t KR, uint32_t RGW) {                      \
-    stream_gemm<F, NMAT, AF, 8, 2>(Ax, rs, W0, W1, C, T, N, K, KR, RGW);                    \
-  }                                                                                         \
-  extern "C" __global__ __launch_bounds__(512) void NAME##_t3_k(                            \
-      const _Float16* Ax, const float* rs, const uint8_t* W0, const uint8_t* W1, float* C,  \
-      uint32_t T, uint32_t N, uint32_t K, uint32_t KR, uint32_t RGW) {                      \
-    stream_gemm<F, NMAT, AF, 8, 3>(Ax, rs, W0, W1, C, T, N, K, KR, RGW);                    \
+    stream_gemm<F, NMAT, AF, TG>(Ax, rs, W0, W1, C, T, N, K, KR, RGW);                      \
   }
-GH_SGEMM(gh_pf_sgemm_q4, SQ4, 1, false)
-GH_SGEMM(gh_pf_sgateup_q4, SQ4, 2, false)
-GH_SGEMM(gh_pf_sgemm_q8, SQ8, 1, false)
-GH_SGEMM(gh_pf_sgateup_q8, SQ8, 2, false)
-GH_SGEMM(gh_pf_sgemm_bf16, SBf16, 1, false)
-GH_SGEMM(gh_pf_sgateup_bf16, SBf16, 2, false)
-GH_SGEMM(gh_pf_sgemm_q4_f, SQ4, 1, true)
-GH_SGEMM(gh_pf_sgateup_q4_f, SQ4, 2, true)
-GH_SGEMM(gh_pf_sgemm_q8_f, SQ8, 1, true)
-GH_SGEMM(gh_pf_sgateup_q8_f, SQ8, 2, true)
-GH_SGEMM(gh_pf_sgemm_bf16_f, SBf16, 1, true)
-GH_SGEMM(gh_pf_sgateup_bf16_f, SBf16, 2, true)
+#define GH_SGEMM_TG2(FMT, F, TG)                      \
+  GH_SGEMM_TG(gh_pf_sgemm_##FMT, F, 1, false, TG)     \
+  GH_SGEMM_TG(gh_pf_sgemm_##FMT##_f, F, 1, true, TG)
+#define GH_SGATEUP_TG2(FMT, F, TG)                    \
+  GH_SGEMM_TG(gh_pf_sgateup_##FMT, F, 2, false, TG)   \
+  GH_SGEMM_TG(gh_pf_sgateup_##FMT##_f, F, 2, true, TG)
+// (the lengths that the host streams: longer ones take the wide tile)
+GH_SGEMM_TG2(q4, SQ4, 0) GH_SGEMM_TG2(q4, SQ4, 1) GH_SGEMM_TG2(q4, SQ4, 2) GH_SGEMM_TG2(q4, SQ4, 3)
+GH_SGEMM_TG2(q8, SQ8, 0) GH_SGEMM_TG2(q8, SQ8, 1) GH_SGEMM_TG2(q8, SQ8, 2) GH_SGEMM_TG2(q8, SQ8, 3)
+GH_SGEMM_TG2(bf16, SBf16, 0) GH_SGEMM_TG2(bf16, SBf16, 1) GH_SGEMM_TG2(bf16, SBf16, 2)
+GH_SGATEUP_TG2(q4, SQ4, 0) GH_SGATEUP_TG2(q4, SQ4, 1) GH_SGATEUP_TG2(q4, SQ4, 2) GH_SGATEUP_TG2(q4, SQ4, 3)
+GH_SGATEUP_TG2(q8, SQ8, 0) GH_SGATEUP_TG2(q8, SQ8, 1) GH_SGATEUP_TG2(q8, SQ8, 2) GH_SGATEUP_TG2(q8, SQ8, 3)
+GH_SGATEUP_TG2(bf16, SBf16, 0) GH_SGATEUP_TG2(bf16, SBf16, 1)
 
 // ---------------------------------------------------------------------------
 // Row-wise x prologue for T tokens (the batched form of the decode GEMVs'

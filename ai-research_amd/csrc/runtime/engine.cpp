@@ -375,40 +375,65 @@ gh_status launch_attention(gh_context* ctx, const AttnLaunch& L) {
 }
 
 namespace {
-// The weight-streaming GEMM of a short batch (T <= 16, gh_pf_sgemm_* /
-// gh_pf_sgateup_*): workgroups of 4 waves over 4 RGW row groups of 16 and a
-// K slice of KR quant blocks.  LDS holds the slice's T activation rows (128 KR
-// + 16 bytes each) and each wave's weight set rows (16 rows of SB blocks + 16
-// bytes per matrix: SB = 16 for Q4/Q8, 8 for bf16).  Slices of 16 blocks and
-// about one round of resident workgroups (RGW row groups per wave so that
-// the grid is near the CUs' workgroup slots) measured fastest at the 12B
-// shapes (16 tokens, Q4: QKV 8192 x 3840 at RGW 2, o 3840 x 4096 at 1,
-// gate+up 2 x 15360 x 3840 and down 3840 x 15360 at 4); wider slices (24, 32)
-// and 2-4x the workgroups were slower.  GH_PF_STREAM="kr,rgw" forces both
-// (kr a multiple of 4, at most 32).  af: A is the f32 rows (Ax) and the
-// kernel splits each slice itself (gh_pf_*_f_k; rs unused).
-// LDS of one workgroup of the streamed GEMM: T staged token rows of a
-// kr-block slice, then the set rows of each of its waves (4 waves for up to
-// 16 tokens, 8 for 17-48), plus 256 bytes for its static per-token slice
-// scales.
-uint32_t stream_lds(gh_quant_mode mode, bool pair, uint32_t T, uint32_t kr) {
-  const uint32_t block_bytes = mode == GH_QUANT_Q8 ? 36u : mode == GH_QUANT_NONE ? 64u : 20u;
-  const uint32_t set_blocks = mode == GH_QUANT_NONE ? 8u : 16u;
-  const uint32_t wave_bytes = 16u * (set_blocks * block_bytes + 16u);
-  const uint32_t nw = T <= 16 ? 4u : 8u;
-  return T * (128u * kr + 16u) + nw * (pair ? 2u : 1u) * wave_bytes + 256u;
+// ---- the weight-streaming GEMM of a short batch (gh_pf_sgemm_* /
+// gh_pf_sgateup_*): workgroups of nw waves over nw rgw units of 16 rows (of each
+// matrix of a gate/up pair) and a K slice of kr quant blocks, whose T activation
+// rows (128 kr + 16 bytes each) are staged in LDS.
+struct StreamCut {
+  uint32_t kr = 0, rgw = 1, nw = 8;
+};
+
+uint32_t stream_lds(uint32_t T, uint32_t kr) { return T * (128u * kr + 16u); }
+
+// Widest slice: what LDS holds beside the static slice scales, and what a
+// thread's registers hold while it splits f32 rows (StreamStage in
+// prefill.hip; 4 kr groups per token).
+uint32_t stream_kr_max(const gh_context* ctx, uint32_t T, uint32_t nw) {
+  const uint32_t regs = T <= 16 ? 10 * nw : T <= 32 ? 5 * nw : 4 * nw;
+  const uint32_t lds = ((uint32_t)ctx->max_lds - 256u - 16u * T) / (128u * T);
+  return std::min(regs, lds) & ~3u;
 }
 
-// The streamed GEMM's slice width in quant blocks: 16 (or all of K); for
-// more than 32 tokens, else 12 or 8 if the staged rows fit in LDS then (and
-// the slices stay at 64 or fewer); 0 when none does.  Narrower slices multiply
-// the planes: the bf16 gate/up pair of 40 tokens in 4-block slices (30
-// planes) took the prompt from 9.9 to 14.7 ms.
-uint32_t stream_kr(const gh_context* ctx, gh_quant_mode mode, bool pair, uint32_t T, uint32_t nb) {
-  const uint32_t narrowest = T <= 32 ? std::min(16u, nb) : std::min(8u, nb);
-  for (uint32_t kr = std::min(16u, nb); kr >= narrowest; kr -= 4)
-    if (stream_lds(mode, pair, T, kr) <= ctx->max_lds && (nb + kr - 1) / kr <= 64) return kr;
-  return 0;
+// The cut with the least streaming per CU (rounds of workgroups times waves
+// times sets of a wave), then the least staging and plane traffic.  Against
+// every cut measured for 166 products (three weight modes, 8 shapes of 2048 -
+// 15360 rows by 1536 - 15360, 3 - 48 tokens) this takes one 1.1% behind the
+// best in the mean, 12% at worst.  Four waves serve narrow products: W_o of 16
+// tokens (3840 x 4096) 11.4 us on 120 workgroups of eight waves, 10.0 on 240 of
+// four.
+StreamCut stream_cut(const gh_context* ctx, gh_quant_mode mode, bool pair, uint32_t T, uint32_t N,
+                     uint32_t nb) {
+  const uint32_t cus = (uint32_t)ctx->num_cus, units = (N + 15) / 16;
+  StreamCut best;
+  if (const char* env = getenv("GH_PF_STREAM")) {
+    unsigned kr = 0, rgw = 0, nw = 8;
+    if (sscanf(env, "%u,%u,%u", &kr, &rgw, &nw) >= 2 && kr >= 4 && kr % 4 == 0 && (nw == 4 || nw == 8) &&
+        std::min(kr, nb) <= stream_kr_max(ctx, T, nw) && (nb + kr - 1) / kr <= 64 && rgw >= 1 && rgw <= 8)
+      return StreamCut{std::min(kr, nb), rgw, nw};
+  }
+  // blocks of a register set; the weight of a wave's sets of one unit
+  const uint32_t sb = mode == GH_QUANT_NONE ? 8u : 16u;
+  const double passes = pair ? 8.0 : 4.0;
+  double least = 0;
+  for (uint32_t nw = 4; nw <= 8; nw += 4) {
+    const uint32_t krmax = std::min(stream_kr_max(ctx, T, nw), nb);
+    if (krmax < 4) continue;
+    for (uint32_t nz = (nb + krmax - 1) / krmax; nz <= std::min(64u, nb / 4); nz++) {
+      const uint32_t kr = ((nb + nz - 1) / nz + 3) & ~3u;
+      if (kr > krmax || (nb + kr - 1) / kr != nz) continue;
+      for (uint32_t rgw = 1; rgw <= 8; rgw++) {
+        const uint32_t wgs = ((units + nw * rgw - 1) / (nw * rgw)) * nz;
+        const double rounds = (wgs + cus - 1) / cus;
+        double cost = rounds * (6.45 + 0.02 * kr * T / nw + passes * nw * rgw * ((kr + sb - 1) / sb));
+        if (nz > 1) cost += 0.3 + 0.6 * nz * (pair ? 2 : 1) * T * (double)N * 8 / 4e6;
+        if (best.kr == 0 || cost < least) {
+          least = cost;
+          best = StreamCut{kr, rgw, nw};
+        }
+      }
+    }
+  }
+  return best;
 }
 
 gh_status launch_prefill_stream(gh_context* ctx, gh_quant_mode mode, const void* W0,
@@ -417,37 +442,14 @@ gh_status launch_prefill_stream(gh_context* ctx, gh_quant_mode mode, const void*
                                 uint32_t* nplanes, bool af) {
   const bool pair = W1 != nullptr;
   const uint32_t nmat = pair ? 2u : 1u;
-  const uint32_t nb = K / 32, cus = (uint32_t)ctx->num_cus, rgs = (N + 15) / 16;
-  // waves per workgroup; 16-token groups per wave
-  const uint32_t nw = T <= 16 ? 4u : 8u, tg = T <= 16 ? 1u : T <= 32 ? 2u : 3u;
-  auto lds_of = [&](uint32_t kr) { return stream_lds(mode, pair, T, kr); };
-  uint32_t KR = stream_kr(ctx, mode, pair, T, nb);
-  if (KR == 0) return fail(GH_ERR_UNSUPPORTED, "prefill GEMM: stream slice exceeds LDS");
+  const uint32_t nb = K / 32, cus = (uint32_t)ctx->num_cus;
+  const StreamCut cut = stream_cut(ctx, mode, pair, T, N, nb);
+  if (cut.kr == 0) return fail(GH_ERR_UNSUPPORTED, "prefill GEMM: stream slice exceeds LDS");
+  uint32_t KR = cut.kr, RGW = cut.rgw;
+  const uint32_t nz = (nb + KR - 1) / KR, units = (N + 15) / 16;
   const std::string kname = std::string(pair ? "gh_pf_sgateup_" : "gh_pf_sgemm_") +
                             (mode == GH_QUANT_Q8 ? "q8" : mode == GH_QUANT_NONE ? "bf16" : "q4") +
-                            (af ? "_f" : "") + (tg == 3 ? "_t3_k" : tg == 2 ? "_t2_k" : "_k");
-  // RGW: the grid sized for the workgroups LDS lets a CU hold, at most two.
-  // Sizing it for the 3-4 a CU could hold with a one-matrix set buffer
-  // (fewer row groups per wave, so shorter streams) measured slower: gate+up
-  // 46.3 against 36.0 us, QKV 20.4 against 16.1 (16 tokens, f32 input, plane
-  // sums included); and that buffer itself, at the same grid, 37.0 against
-  // 35.1 us for the gate+up.
-  const uint32_t per_cu = std::max(1u, std::min(2u, (uint32_t)(ctx->max_lds / lds_of(KR))));
-  const uint32_t slots = per_cu * cus, nz16 = (nb + KR - 1) / KR;
-  uint32_t RGW = (uint32_t)(((uint64_t)rgs * nz16 + (nw / 2) * slots) / (nw * (uint64_t)slots));
-  RGW = std::max(1u, std::min(8u, RGW));
-  if (const char* env = getenv("GH_PF_STREAM")) {
-    unsigned kr = 0, rgw = 0;
-    if (sscanf(env, "%u,%u", &kr, &rgw) == 2 && kr >= 4 && kr % 4 == 0 && kr <= 32 &&
-        lds_of(std::min(kr, nb)) <= ctx->max_lds && rgw >= 1 && rgw <= 8) {
-      KR = std::min(kr, nb);
-      RGW = rgw;
-    }
-  }
-  const uint32_t nz = (nb + KR - 1) / KR;
-  if (nz > 64) return fail(GH_ERR_UNSUPPORTED, "prefill GEMM: more than 64 K slices");
-  const unsigned lds = lds_of(KR);
-  if (lds > ctx->max_lds) return fail(GH_ERR_UNSUPPORTED, "prefill GEMM: stream slice exceeds LDS");
+                            (af ? "_f_t" : "_t") + std::to_string(T <= 8 ? 0 : (T + 15) / 16) + "_k";
   float* out = C;
   if (nz > 1) {
     const size_t need = (size_t)nz * nmat * T * N * sizeof(float);
@@ -458,9 +460,8 @@ gh_status launch_prefill_stream(gh_context* ctx, gh_quant_mode mode, const void*
   const void* W1a = pair ? W1 : W0;
   void* args[] = {const_cast<void**>(&Ax), const_cast<float**>(&rs), const_cast<void**>(&W0),
                   const_cast<void**>(&W1a), &out, &T, &N, &K, &KR, &RGW};
-  const dim3 grid((rgs + nw * RGW - 1) / (nw * RGW), 1, nz);
-  // dynamic LDS: all of it but the static slice scales' share
-  gh_status st = ctx->launch(kname, grid, dim3(64 * nw), lds - 256u, args);
+  const dim3 grid((units + cut.nw * RGW - 1) / (cut.nw * RGW), 1, nz);
+  gh_status st = ctx->launch(kname, grid, dim3(64 * cut.nw), stream_lds(T, KR), args);
   if (planes) {
     *planes = nz > 1 ? out : C;
     *nplanes = nz;
@@ -474,18 +475,19 @@ gh_status launch_prefill_stream(gh_context* ctx, gh_quant_mode mode, const void*
 }
 
 // Short batches stream the weights (16-byte pieces of 4-block runs: K a
-// multiple of 128, rows 16-byte aligned): up to 16 tokens, and up to 48 (bf16
-// rows: 40) when the 8-wave workgroup's LDS fits (GH_PF_STREAM_MAX lowers the
-// limit).  Measured on the 12B shape against the tile GEMMs, prompts of
-// 33 / 40 / 48 tokens: Q4 9.3 / 9.4 / 9.5 -> 7.2 / 7.9 / 8.0 ms, Q8 (33, 48)
-// 10.2 / 10.5 -> 8.4 / 9.4, bf16 9.5 / 9.6 / 9.9 -> 8.8 / 9.0 / 10.0.
-bool stream_ok(const gh_context* ctx, gh_quant_mode mode, uint32_t T, uint32_t K, const void* W0,
-               const void* W1) {
-  uint32_t tmax = mode == GH_QUANT_NONE ? 40u : 48u;
+// multiple of 128, rows 16-byte aligned) as far as that beats the wide tile
+// (GH_PF_STREAM_MAX lowers the limits).  us, streamed / wide, at the limit and
+// past it: Q4 gate/up 2 x 15360 x 3840 of 40 tokens 52.6 / 52.8, 48 tokens 54.4
+// / 53.5; bf16 gate/up of 16 tokens 53-56 / 53, 32 tokens 69 / 58; Q4 down of
+// 48 tokens 33 / 36; bf16 down of 32 tokens 38 / 39, 40 tokens 44 / 40.
+bool stream_ok(const gh_context* ctx, gh_quant_mode mode, uint32_t T, uint32_t N, uint32_t K,
+               const void* W0, const void* W1) {
+  const bool bf16 = mode == GH_QUANT_NONE;
+  uint32_t tmax = W1 ? (bf16 ? 16u : mode == GH_QUANT_Q4 ? 40u : 48u) : (bf16 ? 32u : 48u);
   if (const char* env = getenv("GH_PF_STREAM_MAX")) tmax = std::min(tmax, (uint32_t)atoi(env));
   return T <= tmax && K % 128 == 0 &&
          !((reinterpret_cast<uintptr_t>(W0) | reinterpret_cast<uintptr_t>(W1 ? W1 : W0)) & 15) &&
-         stream_kr(ctx, mode, W1 != nullptr, T, K / 32) != 0 &&
+         stream_cut(ctx, mode, W1 != nullptr, T, N, K / 32).kr != 0 &&
          getenv("GH_PF_NO_STREAM") == nullptr;
 }
 
@@ -613,7 +615,7 @@ gh_status launch_prefill_gemm_split(gh_context* ctx, gh_quant_mode mode, const v
                                 "(16-byte for bf16 rows)");
   const bool pair = W1 != nullptr;
   if (pair && planes) return fail(GH_ERR_INVALID, "prefill GEMM: unsummed planes of a gate/up pair");
-  if (stream_ok(ctx, mode, T, K, W0, W1))
+  if (stream_ok(ctx, mode, T, N, K, W0, W1))
     return launch_prefill_stream(ctx, mode, W0, W1, Ax, rs, C, T, N, K, planes, nplanes, false);
   // Longer batches take the wide tile, 1.02-1.75x the speed of the tiles below
   // wherever both were measured (wide_shape).  Those stay for K that is no
@@ -763,7 +765,7 @@ gh_status launch_prefill_gemm(gh_context* ctx, gh_quant_mode mode, const void* W
     return fail(GH_ERR_INVALID, "prefill GEMM: W null or misaligned (4 bytes; 16 for bf16 rows)");
   if (W1 && planes) return fail(GH_ERR_INVALID, "prefill GEMM: unsummed planes of a gate/up pair");
   // a short batch's streamed GEMM splits the f32 rows as it stages them
-  if (stream_ok(ctx, mode, T, K, W0, W1))
+  if (stream_ok(ctx, mode, T, N, K, W0, W1))
     return launch_prefill_stream(ctx, mode, W0, W1, A, nullptr, C, T, N, K, planes, nplanes, true);
   const size_t ax_bytes = (size_t)T * K * 4;  // 2 K halves per row
   gh_status st = ctx->ensure_zeroed(&ctx->half_scratch, &ctx->half_scratch_bytes,

@@ -249,6 +249,38 @@ def test_prefill_stream_slices(gpu, monkeypatch, T, shape):
                  nr.gelu64(a64 @ gdeq.T) * (a64 @ udeq.T), what="streamed GeGLU, slices %s" % shape)
 
 
+# The streamed GEMM's token groups at their edges (up to 8 tokens: hi and lo in
+# one MFMA; up to 16, 32 and 48), four- and eight-wave workgroups ("kr,rgw,nw":
+# quant blocks of a slice, units of 16 rows per wave, waves), one unsplit slice,
+# slices that end in a partial register set, waves past N.  Bound as in
+# test_prefill_wide_tiles: the activations enter at 22 (16) bits.
+@pytest.mark.parametrize("mode", [gh.QUANT_Q4, gh.QUANT_Q8, gh.QUANT_NONE])
+@pytest.mark.parametrize("T,N,K,cut", [
+    (1, 33, 128, "4,1,8"), (8, 200, 640, "12,1,4"), (8, 130, 1280, "40,2,4"), (9, 47, 640, "20,1,8"),
+    (16, 300, 2560, "80,1,8"), (15, 100, 1280, "40,1,4"), (17, 90, 1280, "20,3,4"),
+    (32, 140, 1280, "40,1,8"), (33, 70, 1024, "32,2,8"), (48, 260, 640, "16,1,4"),
+    (48, 50, 640, "20,1,8")])
+def test_prefill_stream_cuts(gpu, monkeypatch, mode, T, N, K, cut):
+    monkeypatch.setenv("GH_PF_STREAM", cut)
+    rtol = 1e-3 if mode == gh.QUANT_NONE else 2e-5
+    gq, gdeq = quantized(N, K, mode, 394)
+    uq, udeq = quantized(N, K, mode, 395)
+    a = gh.synth_normal(T * K, 1, 396, 0.0, 1.0).reshape(T, K)
+    a64 = np.asarray(a, np.float64)
+    A, C, W, Wu = gpu.upload(a), gpu.alloc((T + 16) * N * 4), gpu.upload(gq), gpu.upload(uq)
+    gpu.fill_u32(C, 0x7FC12345, (T + 16) * N)
+    for pair in (False, True):
+        if pair:
+            gpu.prefill_gate_up_geglu(mode, W, Wu, A, C, T, N, K)
+            ref = nr.gelu64(a64 @ gdeq.T) * (a64 @ udeq.T)
+        else:
+            gpu.prefill_gemm(mode, W, A, C, T, N, K)
+            ref = a64 @ gdeq.T
+        out = C.read(np.uint32, (T + 16) * N).reshape(T + 16, N)
+        assert np.all(out[T:] == 0x7FC12345)  # nothing past row T - 1
+        assert_close(out[:T].view(np.float32), ref, rtol=rtol, what="streamed, cut %s" % cut)
+
+
 @pytest.mark.parametrize("N", [320, 203])
 @pytest.mark.parametrize("pair", [False, True])
 @pytest.mark.parametrize("split", ["1", "3", "200"])
