@@ -18,6 +18,9 @@
 
 #include <algorithm>
 #include <cmath>
+#include <functional>
+#include <memory>
+#include <new>
 #include <string>
 #include <vector>
 
@@ -147,7 +150,11 @@ struct gh_model {
 namespace {
 gh_status ensure_prefill(gh_model* m, uint32_t T, uint32_t stride);
 gh_status reset_gates(gh_model* m);
-gh_status prefill_forward(gh_model* m, uint32_t T, bool want_logits);
+gh_status prefill_forward(gh_model* m, uint32_t T, bool want_logits,
+                          const std::function<gh_status()>& lists);
+gh_status prefill_batch(gh_model* m, const float* x, bool x_up, uint32_t T, const uint64_t* clocks,
+                        const uint32_t* slot_idx, const uint32_t* active, uint32_t active_stride,
+                        const uint32_t* n_active, int want_logits, uint32_t* out_token);
 }  // namespace
 
 gh_model::~gh_model() {
@@ -628,13 +635,26 @@ gh_status reset_gates(gh_model* m) {
 
 // Sends the host mirror's layer-0 ring state to the device arrays the ring
 // kernel reads.
-gh_status ring_upload(gh_model* m) {
+// Queues the copy of ring `r`'s layer 0 state; `st` holds it until the copy
+// is done.
+hipError_t ring_queue(gh_model* m, const gh_ring* r, std::vector<uint32_t>* st) {
   const uint32_t n = m->cfg.max_slots;
-  std::vector<uint32_t> st(2 * (size_t)n, 0u);
-  if (m->ring) gh::ring_state(m->ring, 0, st.data(), st.data() + n, n);
-  gh_status s = gh_buffer_write(m->ctx, m->at<uint32_t>(m->ring_clock), st.data(), (size_t)n * 4);
-  if (s == GH_OK) s = gh_buffer_write(m->ctx, m->at<uint32_t>(m->ring_flag), st.data() + n, (size_t)n * 4);
-  return s;
+  st->assign(2 * (size_t)n, 0u);
+  if (r) gh::ring_state(r, 0, st->data(), st->data() + n, n);
+  hipError_t e = hipMemcpyAsync(m->at<uint32_t>(m->ring_clock), st->data(), (size_t)n * 4,
+                                hipMemcpyHostToDevice, m->ctx->stream);
+  if (e == hipSuccess)
+    e = hipMemcpyAsync(m->at<uint32_t>(m->ring_flag), st->data() + n, (size_t)n * 4,
+                       hipMemcpyHostToDevice, m->ctx->stream);
+  return e;
+}
+
+gh_status ring_upload(gh_model* m) {
+  std::vector<uint32_t> st;
+  hipError_t e = ring_queue(m, m->ring, &st);
+  const hipError_t es = hipStreamSynchronize(m->ctx->stream);
+  if (e == hipSuccess) e = es;
+  return e == hipSuccess ? GH_OK : hip_fail(e, "ring state copy");
 }
 
 gh_status rerecord(gh_model* m) {
@@ -989,35 +1009,46 @@ gh_status gh_model_ring_prefill(gh_model* m, const float* x, uint32_t T, uint64_
     return fail(GH_ERR_INVALID, "gh_model_ring_prefill: T is zero or a clock exceeds 2^32");
   const uint32_t total = gh_ring_total_slots(m->ring);
   std::vector<uint64_t> clocks(T);
-  std::vector<uint32_t> slots(T), n(T), lists((size_t)T * total);
+  std::vector<uint32_t> slots(T), n(T);
+  std::unique_ptr<uint32_t[]> lists(new (std::nothrow) uint32_t[(size_t)T * total]);
+  if (!lists) return fail(GH_ERR_ALLOC, "gh_model_ring_prefill: active lists");
   // the lists as the per-token calls would see them: slot activations of the
   // earlier tokens of the batch included, later ones not; a failed call
   // leaves the ring as it was
   gh_ring* r = gh::ring_clone(m->ring);
   if (!r) return fail(GH_ERR_ALLOC, "gh_model_ring_prefill: ring copy");
-  for (uint32_t t = 0; t < T; t++) {
-    clocks[t] = first_clock + t;
-    slots[t] = gh_ring_activate_slot(r, 0, clocks[t]);
-    n[t] = gh_ring_active_slots(r, 0, clocks[t], &lists[(size_t)t * total], total);
-  }
-  // gh_model_prefill advances m->ring as its tokens or chunks finish: keep
+  // the call below advances m->ring as its tokens or chunks finish: keep
   // the state from before the call to put back on failure
   gh_ring* before = gh::ring_clone(m->ring);
   if (!before) {
     gh_ring_destroy(r);
     return fail(GH_ERR_ALLOC, "gh_model_ring_prefill: ring copy");
   }
-  gh_status st = gh_model_prefill(m, x, T, clocks.data(), slots.data(), lists.data(), total,
-                                  n.data(), want_logits, out_token);
-  gh_ring_destroy(st == GH_OK ? before : r);
-  gh_ring_destroy(m->ring);
-  m->ring = st == GH_OK ? r : before;
-  if (st != GH_OK) {
-    const std::string why = gh_last_error();
-    ring_upload(m);
-    return fail(st, why);
+  // A batch whose buffers are there starts its x on the way before its lists
+  // are built: at 512 tokens the copy call takes 150 us, the copy 230, and
+  // the lists and their checks 160.  A batch that runs in parts copies its
+  // rows again, to the same buffer and behind this copy.
+  const bool x_up = T > m->seq_prefill_max && !(m->q_on && want_logits) && m->pf_arena &&
+                    m->pf_cap >= T && m->pf_stride >= total && m->cfg.hidden_size <= 8192 &&
+                    hipMemcpyAsync(m->pf_x, x, (size_t)T * m->cfg.hidden_size * 4,
+                                   hipMemcpyHostToDevice, m->ctx->stream) == hipSuccess;
+  for (uint32_t t = 0; t < T; t++) {
+    clocks[t] = first_clock + t;
+    slots[t] = gh_ring_activate_slot(r, 0, clocks[t]);
+    n[t] = gh_ring_active_slots(r, 0, clocks[t], lists.get() + (size_t)t * total, total);
   }
-  return ring_upload(m);
+  gh_status st = prefill_batch(m, x, x_up, T, clocks.data(), slots.data(), lists.get(), total,
+                               n.data(), want_logits, out_token);
+  gh_ring_destroy(r);
+  if (st == GH_OK) {  // m->ring and the device's copy have taken the batch's activations
+    gh_ring_destroy(before);
+    return GH_OK;
+  }
+  const std::string why = gh_last_error();
+  gh_ring_destroy(m->ring);
+  m->ring = before;
+  ring_upload(m);  // also waits for the copy of x
+  return fail(st, why);
 }
 
 gh_status gh_model_set_quiescence(gh_model* m, float threshold) {
@@ -1046,6 +1077,18 @@ gh_status gh_model_prefill(gh_model* m, const float* x, uint32_t T, const uint64
                            const uint32_t* slot_idx, const uint32_t* active,
                            uint32_t active_stride, const uint32_t* n_active, int want_logits,
                            uint32_t* out_token) {
+  return prefill_batch(m, x, false, T, clocks, slot_idx, active, active_stride, n_active,
+                       want_logits, out_token);
+}
+
+}  // extern "C"
+
+namespace {
+
+// gh_model_prefill; with x_up the copy of x to m->pf_x is already queued.
+gh_status prefill_batch(gh_model* m, const float* x, bool x_up, uint32_t T, const uint64_t* clocks,
+                        const uint32_t* slot_idx, const uint32_t* active, uint32_t active_stride,
+                        const uint32_t* n_active, int want_logits, uint32_t* out_token) {
   if (!m || !x || !clocks || !slot_idx || !active || !n_active || !out_token)
     return fail(GH_ERR_INVALID, "gh_model_prefill: null argument");
   *out_token = 0;
@@ -1062,22 +1105,24 @@ gh_status gh_model_prefill(gh_model* m, const float* x, uint32_t T, const uint64
   // and earlier tokens' slots, and no slot written twice.  A batch that
   // breaks this (a wrapped window: token t still attends to the slot token
   // t + 1 overwrites) runs token by token instead, as does a short one.
-  std::vector<int64_t> writer(c.max_slots, -1);
+  std::vector<uint32_t> writer(c.max_slots, 0u);  // 1 + the token that writes the slot, else 0
   bool conflict = false;
   for (uint32_t t = 0; t < T; t++) {
     if (slot_idx[t] >= c.max_slots || clocks[t] > 0xFFFFFFFFull)
       return fail(GH_ERR_INVALID, "gh_model_prefill: slot or clock out of range");
-    conflict = conflict || writer[slot_idx[t]] >= 0;
-    writer[slot_idx[t]] = t;
+    conflict = conflict || writer[slot_idx[t]] != 0;
+    writer[slot_idx[t]] = t + 1;
   }
   for (uint32_t t = 0; t < T; t++) {
     if (n_active[t] == 0 || n_active[t] > c.max_slots)
       return fail(GH_ERR_INVALID, "gh_model_prefill: active list length out of range");
     const uint32_t* row = active + (size_t)t * active_stride;
+    uint32_t late = 0;
     for (uint32_t i = 0; i < n_active[t]; i++) {
       if (row[i] >= c.max_slots) return fail(GH_ERR_INVALID, "gh_model_prefill: active slot out of range");
-      conflict = conflict || writer[row[i]] > (int64_t)t;
+      late |= writer[row[i]] > t + 1;
     }
+    conflict = conflict || late != 0;
   }
   if (m->ring)
     for (uint32_t t = 0; t < T; t++)
@@ -1091,7 +1136,7 @@ gh_status gh_model_prefill(gh_model* m, const float* x, uint32_t T, const uint64
   // 183).
   if (m->q_on && want_logits) {
     if (T > 1) {
-      gh_status ps = gh_model_prefill(m, x, T - 1, clocks, slot_idx, active, active_stride,
+      gh_status ps = prefill_batch(m, x, false, T - 1, clocks, slot_idx, active, active_stride,
                                       n_active, 0, out_token);
       if (ps != GH_OK) return ps;
     }
@@ -1103,7 +1148,7 @@ gh_status gh_model_prefill(gh_model* m, const float* x, uint32_t T, const uint64
     // staged batches hold at most stage_rows tokens: consecutive chunks
     for (uint32_t t0 = 0; t0 < T; t0 += m->stage_rows) {
       const uint32_t n = std::min(T - t0, m->stage_rows);
-      gh_status cs = gh_model_prefill(m, x + (size_t)t0 * c.hidden_size, n, clocks + t0,
+      gh_status cs = prefill_batch(m, x + (size_t)t0 * c.hidden_size, false, n, clocks + t0,
                                       slot_idx + t0, active + (size_t)t0 * active_stride,
                                       active_stride, n_active + t0,
                                       t0 + n == T ? want_logits : 0, out_token);
@@ -1157,12 +1202,9 @@ gh_status gh_model_prefill(gh_model* m, const float* x, uint32_t T, const uint64
     meta[T + t] = conflict ? nslot + t : slot_idx[t];
     meta[2 * T + t] = n_active[t];
   }
-  std::vector<uint32_t> act((size_t)T * m->pf_stride, 0u);
-  for (uint32_t t = 0; t < T; t++)
-    memcpy(&act[(size_t)t * m->pf_stride], active + (size_t)t * active_stride, (size_t)n_active[t] * 4);
-  hipError_t e = hipMemcpyAsync(m->pf_x, x, (size_t)T * c.hidden_size * 4, hipMemcpyHostToDevice, s);
+  hipError_t e = hipSuccess;
+  if (!x_up) e = hipMemcpyAsync(m->pf_x, x, (size_t)T * c.hidden_size * 4, hipMemcpyHostToDevice, s);
   if (e == hipSuccess) e = hipMemcpyAsync(m->pf_meta, meta.data(), meta.size() * 4, hipMemcpyHostToDevice, s);
-  if (e == hipSuccess) e = hipMemcpyAsync(m->pf_active, act.data(), act.size() * 4, hipMemcpyHostToDevice, s);
   // Grouped attention: the matrix-core kernel when every layer has head_dim
   // 256 and one G = nq / nkv dividing 16 (16 / G tokens per group) and the
   // batch has more than 64 tokens, else the 4-token kernel when every layer
@@ -1195,49 +1237,65 @@ gh_status gh_model_prefill(gh_model* m, const float* x, uint32_t T, const uint64
       gtok = kPfGroup;
     }
   }
+  // The attention's lists, built and copied once layer 0's projection is
+  // queued: no earlier kernel reads them, so the host's pass over them (at 512
+  // tokens some 130k entries) runs while the GPU works.  They live to the end
+  // of this call, as the copies may still read them.
+  std::vector<uint32_t> act, ucount;
+  std::unique_ptr<uint32_t[]> uni;
   m->pf_gkind = 0;
-  std::vector<uint32_t> uni, ucount;
-  if (gkind) {
-    const uint32_t groups = (T + gtok - 1) / gtok;
-    const uint32_t ustride = std::min(gtok * m->pf_stride, nrows);
-    uni.assign((size_t)groups * ustride * 2, 0u);
-    ucount.assign(groups, 0u);
-    std::vector<uint32_t> stamp(nrows, 0u), pos(nrows);
-    bool ok = true;
-    for (uint32_t g = 0; g < groups && ok; g++) {
-      uint32_t* u = &uni[(size_t)g * ustride * 2];
-      uint32_t n = 0;
-      for (uint32_t i = 0; i < gtok && g * gtok + i < T && ok; i++) {
-        const uint32_t t = g * gtok + i;
-        const uint32_t* row = active + (size_t)t * active_stride;
-        for (uint32_t k = 0; k < n_active[t]; k++) {
-          const uint32_t slot = row[k];
-          if (stamp[slot] != g + 1) {
-            stamp[slot] = g + 1;
-            pos[slot] = n;
-            u[2 * n] = slot;
-            u[2 * n + 1] = 1u << i;
-            n++;
-          } else if ((u[2 * pos[slot] + 1] >> i) & 1u) {
-            ok = false;
-            break;
-          } else {
-            u[2 * pos[slot] + 1] |= 1u << i;
+  auto attention_lists = [&]() -> gh_status {
+    hipError_t e = hipSuccess;
+    bool ok = gkind != 0;
+    if (ok) {
+      const uint32_t groups = (T + gtok - 1) / gtok;
+      const uint32_t ustride = std::min(gtok * m->pf_stride, nrows);
+      const size_t words = (size_t)groups * ustride * 2;
+      uni.reset(new (std::nothrow) uint32_t[words]);  // entries past a group's count are not read
+      if (!uni) return fail(GH_ERR_ALLOC, "gh_model_prefill: union lists");
+      ucount.assign(groups, 0u);
+      std::vector<uint32_t> stamp(nrows, 0u), pos(nrows);
+      for (uint32_t g = 0; g < groups && ok; g++) {
+        uint32_t* u = uni.get() + (size_t)g * ustride * 2;
+        uint32_t n = 0;
+        for (uint32_t i = 0; i < gtok && g * gtok + i < T && ok; i++) {
+          const uint32_t t = g * gtok + i;
+          const uint32_t* row = active + (size_t)t * active_stride;
+          for (uint32_t k = 0; k < n_active[t]; k++) {
+            const uint32_t slot = row[k];
+            if (stamp[slot] != g + 1) {
+              stamp[slot] = g + 1;
+              pos[slot] = n;
+              u[2 * n] = slot;
+              u[2 * n + 1] = 1u << i;
+              n++;
+            } else if ((u[2 * pos[slot] + 1] >> i) & 1u) {
+              ok = false;
+              break;
+            } else {
+              u[2 * pos[slot] + 1] |= 1u << i;
+            }
           }
         }
+        ucount[g] = n;
       }
-      ucount[g] = n;
+      if (ok) {
+        m->pf_gkind = gkind;
+        m->pf_gtok = gtok;
+        m->pf_ustride = ustride;
+        e = hipMemcpyAsync(m->pf_union, uni.get(), words * 4, hipMemcpyHostToDevice, s);
+        if (e == hipSuccess)
+          e = hipMemcpyAsync(m->pf_ucount, ucount.data(), ucount.size() * 4, hipMemcpyHostToDevice, s);
+      }
     }
-    if (ok) {
-      m->pf_gkind = gkind;
-      m->pf_gtok = gtok;
-      m->pf_ustride = ustride;
-      if (e == hipSuccess)
-        e = hipMemcpyAsync(m->pf_union, uni.data(), uni.size() * 4, hipMemcpyHostToDevice, s);
-      if (e == hipSuccess)
-        e = hipMemcpyAsync(m->pf_ucount, ucount.data(), ucount.size() * 4, hipMemcpyHostToDevice, s);
+    if (!ok) {  // the per-token kernel reads the lists themselves
+      act.assign((size_t)T * m->pf_stride, 0u);
+      for (uint32_t t = 0; t < T; t++)
+        memcpy(&act[(size_t)t * m->pf_stride], active + (size_t)t * active_stride, (size_t)n_active[t] * 4);
+      e = hipMemcpyAsync(m->pf_active, act.data(), act.size() * 4, hipMemcpyHostToDevice, s);
     }
-  }
+    return e == hipSuccess ? GH_OK : hip_fail(e, "gh_model_prefill: list copies");
+  };
   std::vector<uint8_t> table;
   if (conflict) {  // offsets and row words of every cache, then the pairs
     const size_t nc = 2 * m->layers.size();
@@ -1263,7 +1321,10 @@ gh_status gh_model_prefill(gh_model* m, const float* x, uint32_t T, const uint64
     m->pf_trace_cap = T;
   }
   if (m->trace_on) m->pf_trace_T = T;
-  if ((st = prefill_forward(m, T, want_logits != 0)) != GH_OK) return st;
+  if ((st = prefill_forward(m, T, want_logits != 0, attention_lists)) != GH_OK) {
+    hipStreamSynchronize(s);  // the copies read this call's vectors
+    return st;
+  }
   if (conflict) {
     const size_t nc = 2 * m->layers.size();
     uint8_t* base = m->arena;
@@ -1279,16 +1340,29 @@ gh_status gh_model_prefill(gh_model* m, const float* x, uint32_t T, const uint64
     e = hipMemcpyAsync(m->h_token, m->at<uint32_t>(m->token), 4, hipMemcpyDeviceToHost, s);
     if (e != hipSuccess) return hip_fail(e, "gh_model_prefill: token copy");
   }
-  e = hipStreamSynchronize(s);
+  // the ring's new state goes up behind the layers; the host's takes it once
+  // they are done
+  std::unique_ptr<gh_ring, void (*)(gh_ring*)> ring(gh::ring_clone(m->ring), gh_ring_destroy);
+  std::vector<uint32_t> ring_words;
+  if (ring) {
+    for (uint32_t t = 0; t < T; t++) gh_ring_activate_slot(ring.get(), 0, clocks[t]);
+    e = ring_queue(m, ring.get(), &ring_words);
+  }
+  const hipError_t es = hipStreamSynchronize(s);
+  if (e == hipSuccess) e = es;
   if (e != hipSuccess) return hip_fail(e, "gh_model_prefill");
   m->hidden_final = want_logits ? m->x1 : kNone;
   if (want_logits) *out_token = m->h_token[0];
-  if (m->ring) {
-    for (uint32_t t = 0; t < T; t++) gh_ring_activate_slot(m->ring, 0, clocks[t]);
-    return ring_upload(m);
+  if (ring) {
+    gh_ring_destroy(m->ring);
+    m->ring = ring.release();
   }
   return GH_OK;
 }
+
+}  // namespace
+
+extern "C" {
 
 gh_status gh_model_embed(gh_model* m, uint32_t token, float* x_host) {
   if (!m || !x_host) return fail(GH_ERR_INVALID, "gh_model_embed: null argument");
@@ -1385,7 +1459,10 @@ gh_status launch_pf_norm(gh_model* m, uint32_t T, const float* R, const float* w
                         dim3(narrow ? 512 : 1024), 0, args);
 }
 
-gh_status prefill_forward(gh_model* m, uint32_t T, bool want_logits) {
+// The layers of one batch.  `lists` uploads the attention's lists and sets
+// m->pf_gkind; it is called once layer 0's QKV projection is queued.
+gh_status prefill_forward(gh_model* m, uint32_t T, bool want_logits,
+                          const std::function<gh_status()>& lists) {
   gh_context* ctx = m->ctx;
   const gh_model_config& c = m->cfg;
   const uint32_t H = c.hidden_size, I = c.intermediate_size;
@@ -1433,6 +1510,7 @@ gh_status prefill_forward(gh_model* m, uint32_t T, bool want_logits) {
                                             rope4 ? &qkv_planes : nullptr,
                                             rope4 ? &qkv_nz : nullptr)) != GH_OK)
       return st;
+    if (l == 0 && (st = lists()) != GH_OK) return st;
     // 3. q/k norm + RoPE in place, K/V into the caches, then attention
     AttnArgs a{};
     a.q = m->pf_qkv;

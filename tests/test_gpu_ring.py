@@ -124,3 +124,35 @@ def test_ring_prefill_lists_and_wrapped_batches(gpu):
     finally:
         md.close()
         mh.close()
+
+
+@pytest.mark.parametrize("A,W,R,T", [(4, 60, 6, 40), (2, 300, 3, 297), (4, 16, 4, 70)])
+def test_ring_prefill_in_kept_buffers(gpu, A, W, R, T):
+    """A prompt whose rows go up before its lists are built (the buffers are
+    there from an earlier call) against the same prompt on a new model: the
+    batched kernels, the grouped lists, and a wrapped window in parts."""
+    cfg = _cfg(A + W + R)
+    kept, new = (gh.Model(gpu, cfg, seed=4) for _ in range(2))
+    try:
+        xs = np.stack([kept.embed((5 * t + 1) % cfg.vocab_size) for t in range(2 * T)])
+        kept.ring_init(A, W, R)
+        kept.ring_prefill(xs[T:], 0, False)
+        kept.ring_init(A, W, R)
+        new.ring_init(A, W, R)
+        assert kept.ring_prefill(xs[:T], 0, True) == new.ring_prefill(xs[:T], 0, True)
+        ring = gh.Ring(1, A, W, R)
+        for c in range(T):
+            ring.activate_slot(0, c)
+        live = set(ring.active_slots(0, T - 1).tolist())
+        for m in (kept, new):
+            flags = m.read(-1, gh.T_RING_FLAGS, np.uint32)
+            assert live <= set(np.flatnonzero(flags).tolist())
+        for t in (gh.T_LOGITS, gh.T_RING_CLOCKS, gh.T_RING_FLAGS):
+            dt = np.float32 if t == gh.T_LOGITS else np.uint32
+            assert np.array_equal(kept.read(-1, t, dt), new.read(-1, t, dt))
+        assert kept.forward_clock(xs[T], T) == new.forward_clock(xs[T], T)
+        assert np.array_equal(kept.read(-1, gh.T_LOGITS, np.float32),
+                              new.read(-1, gh.T_LOGITS, np.float32))
+    finally:
+        kept.close()
+        new.close()

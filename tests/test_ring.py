@@ -48,3 +48,30 @@ def test_ring_matches_oracle_random():
             q = max(q, 0)
             assert np.array_equal(g.active_slots(0, q), o.active_slots(0, q))
             assert g.slot_index(q) == o.slot_index(q)
+
+
+def test_ring_lists_by_room():
+    """Lists cut by the caller's room: the first `cap` entries of the whole
+    list, its full length returned, nothing written past the room; over rings
+    whose tiers are no multiple of eight and windows that are empty in part."""
+    rng = np.random.default_rng(7)
+    for A, W, R in [(32, 512, 96), (3, 13, 5), (0, 24, 0), (9, 8, 1)]:
+        for filled in (0, 1, W // 2, W + A):
+            g = gh.Ring(1, A, W, R)
+            o = orc.Ring(1, 1, A, W, R)
+            for c in range(filled):
+                if rng.random() < 0.8:
+                    g.activate_slot(0, c)
+                    o.activate_slot(0, c)
+            for rank in range(0, R, 3):
+                c = int(rng.integers(0, 2 * W))
+                g.activate_recall(0, rank, c)
+                o.write_recall_kv(0, rank, np.zeros(1, np.float32), np.zeros(1, np.float32), c)
+            for q in (0, filled // 2, max(filled - 1, 0), filled + W // 2):
+                want = o.active_slots(0, q)
+                for cap in (0, 1, 7, 8, 9, len(want), g.total_slots):
+                    out = np.full(cap + 8, 0xFFFFFFFF, np.uint32)
+                    n = gh.lib().gh_ring_active_slots(g.h, 0, q, gh._ptr(out), cap)
+                    assert n == len(want)
+                    assert np.array_equal(out[:min(n, cap)], want[:cap])
+                    assert (out[cap:] == 0xFFFFFFFF).all()
