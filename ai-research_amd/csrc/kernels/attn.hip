@@ -1103,15 +1103,25 @@ extern "C" __global__ __launch_bounds__(ATT_NT) void gh_pf_attn_merge_k(AttnArgs
 //   O^T (256 dims x 16 columns) += V^T . P^T   64 x v_mfma_f32_16x16x4_f32
 // with the online softmax in between.  Operand mapping (lane l, column
 // l % 16, lane group l / 16):
-//   K . Q^T: the k index of step (j, c) is dim (l/16)*64 + 4j + c, so a lane
-//     loads 64 contiguous floats of its K row (slot l % 16 of the tile) and
-//     reads the same dims of column l % 16's query from LDS.  The result
-//     lands as S[column l % 16][slot 4*(l/16) + r], r = 0..3 --
+//   K . Q^T: the k index of step (j, c) is dim 16 j + 4 (l/16) + c.  The
+//     wave's K tile comes by direct loads to LDS, a whole row of 1 KB each,
+//     its 16-byte pieces swizzled by the slot so that the operand reads (slot
+//     l % 16 of the tile) meet no bank twice; the query operand is in LDS in
+//     operand order.  The result lands as S[column l % 16][slot 4*(l/16) + r],
+//     r = 0..3 --
 //   which is the B operand of V^T . P^T when the k index of step r is slot
 //     4*(l/16) + r: the probabilities feed the second product without a
-//     shuffle.  Its A operand row i of output tile t is dim 16 i + t, so a
-//     lane loads 16 contiguous floats (dims 16*(l%16) ..) of each of its 4
-//     V rows; the result O[column l%16][16*(4*(l/16) + r) + t] sits in o[t][r].
+//     shuffle.  Its A operand row i of output tile t is dim 64 (t/4) + 4 i +
+//     t % 4, so the 16 lanes of a group load 256 contiguous bytes of a V row;
+//     the result O[column l%16][64 (t/4) + 4*(4*(l/16) + r) + t % 4] sits in
+//     o[t][r].
+// What bounds it: the matrix products of a two-wave SIMD (14 us of a
+// 512-token prompt of 16 / 8 heads; a second pass over the same tiles takes
+// 26) and 9 us of prologue, merge and launch.  With each lane loading 256 bytes
+// of its own K row (16 bytes from each of 16 rows per load) the K loads alone
+// cost 12 us: 44.6 -> 39.2 us at 512 tokens, 34.6 -> 30.0 at 300, 14.4 -> 12.9
+// at 128, 13.2 -> 12.5 at 72.  Eight waves per workgroup, one workgroup per CU,
+// took 43.5.
 // The row max and row sum of the softmax reduce over r in the lane and over
 // the 4 lane groups with lane swaps, so every lane of a column holds the same
 // (m, l).  The waves merge through LDS in wave order and write each token's
@@ -1145,21 +1155,30 @@ __device__ __forceinline__ void pfm_entries(const uint32_t* list, uint32_t S, ui
 #pragma unroll
   for (int r = 0; r < 4; r++) {
     const uint32_t i = e0 + 4 * quad + r, ic = min(i, S - 1);
-    e.vslot[r] = list[2 * ic];
-    e.vmask[r] = i < S ? list[2 * ic + 1] : 0u;
+    const uint2 v = *reinterpret_cast<const uint2*>(list + 2 * ic);
+    e.vslot[r] = v.x;
+    e.vmask[r] = i < S ? v.y : 0u;
   }
 }
 
+// 16 bytes per lane from base + off to LDS byte lds + 16 * lane.
+__device__ __forceinline__ void pfm_load_lds16(uint32_t off, const void* base, uint32_t lds) {
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off),
+               "s"(base), "s"(lds)
+               : "memory");
+}
+
 extern "C" __global__ __launch_bounds__(ATT_NT, 2) void gh_pf_attn_m_k(AttnArgs a) {
-  // 64 KB: the query operand (16 steps x 64 lanes of float4) during the
-  // loop, then the waves' o registers ([wave][64 regs][64 lanes]) for the merge
-  __shared__ float4 smem4[ATT_WAVES * 64 * 64 / 4];
-  __shared__ float wm[ATT_WAVES][16], wl[ATT_WAVES][16];
-  float4* qs4 = smem4;
-  float* wo = reinterpret_cast<float*>(smem4);
+  // a K tile per wave and the query operand (16 steps x 64 lanes of float4);
+  // after the loop the waves' o registers and (m, l) take their places
+  __shared__ float4 smem4[ATT_WAVES * 1024 + 1024];
+  float4* qs4 = smem4 + ATT_WAVES * 1024;
+  float* wm = reinterpret_cast<float*>(qs4);  // [wave][16]
+  float* wl = wm + ATT_WAVES * 16;
 
   const uint32_t G = a.nq / a.nkv;
-  const uint32_t tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint32_t tid = threadIdx.x, lane = tid & 63;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t col = lane & 15, quad = lane >> 4;
   const size_t kv_dim = (size_t)a.nkv * PFM_D;
   // group order: the first half of blockIdx.y runs the longest groups in
@@ -1172,23 +1191,34 @@ extern "C" __global__ __launch_bounds__(ATT_NT, 2) void gh_pf_attn_m_k(AttnArgs 
   const uint32_t* list = a.active + (size_t)grp * a.active_stride;
   const uint32_t ntiles = (S + 15) / 16;
 
-  // 1. query columns into LDS in operand order: qs4[j * 64 + l] = dims
-  //    (l/16)*64 + 4j .. +4 of column l % 16 (zeros past the last token)
+  // 1. entries of this wave's first two tiles (indices clamped into the list,
+  //    so every load below is unconditional and in bounds, and masks past the
+  //    end are zero); the first K tile's load
+  PfmEntries cur, nxt;
+  pfm_entries(list, S, wave, col, quad, cur);
+  pfm_entries(list, S, wave + ATT_WAVES, col, quad, nxt);
+  const float* kb = a.k_cache + (size_t)kvh * PFM_D;
+  const float* vb = a.v_cache + (size_t)kvh * PFM_D + col * 4;
+  const uint32_t k_lds = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)smem4 + wave * 16384;
+  auto load_k = [&](uint32_t kslot) {
+#pragma unroll
+    for (int j = 0; j < 16; j++) {
+      const uint32_t slot = __builtin_amdgcn_readlane(kslot, j);
+      pfm_load_lds16(16 * (lane ^ j), kb + (size_t)slot * kv_dim, k_lds + 1024 * j);
+    }
+  };
+  load_k(cur.kslot);
+  //    query columns into LDS in operand order: qs4[j * 64 + l] = dims
+  //    16 j + 4 (l/16) .. +4 of column l % 16 (zeros past the last token)
   for (uint32_t i = tid; i < 16 * 64; i += ATT_NT) {
     const uint32_t j = i >> 6, ln = i & 63, c = ln & 15;
     const uint32_t t = t0 + c / G, g = c % G;
     float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
     if (t < a.n_tokens)
       v = *reinterpret_cast<const float4*>(a.q + (size_t)t * a.q_stride +
-                                           (size_t)(kvh * G + g) * PFM_D + (ln >> 4) * 64 + 4 * j);
+                                           (size_t)(kvh * G + g) * PFM_D + 16 * j + (ln >> 4) * 4);
     qs4[i] = v;
   }
-  // entries of this wave's first two tiles (indices clamped into the list, so
-  // every load below is unconditional and in bounds, and masks past the end
-  // are zero)
-  PfmEntries cur, nxt;
-  pfm_entries(list, S, wave, col, quad, cur);
-  pfm_entries(list, S, wave + ATT_WAVES, col, quad, nxt);
   __syncthreads();
 
   // 2. the wave's tiles: scores, online softmax, weighted V
@@ -1197,62 +1227,33 @@ extern "C" __global__ __launch_bounds__(ATT_NT, 2) void gh_pf_attn_m_k(AttnArgs 
 #pragma unroll
   for (int t = 0; t < 16; t++) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   float m = -INFINITY, l = 0.f;
-  const float* kb = a.k_cache + (size_t)kvh * PFM_D + quad * 64;
-  const float* vb = a.v_cache + (size_t)kvh * PFM_D + col * 16;
-  // The first half of tile i + 4's K rows loads while tile i's V . P
-  // products run, the second half at the top of its iteration, and its V
-  // rows once the first half's score products have freed their registers.
-  // This keeps a wave within 256 registers (two waves per SIMD).
-  float4 kr[16], vr[4][4];
-  {
-    const float4* kp = reinterpret_cast<const float4*>(kb + (size_t)cur.kslot * kv_dim);
-#pragma unroll
-    for (int j = 0; j < 8; j++) kr[j] = kp[j];
-  }
+  const float4* kt = smem4 + wave * 1024 + col * 64;
   for (uint32_t tile = wave; tile < ntiles; tile += ATT_WAVES) {
-    {
-      const float4* kp = reinterpret_cast<const float4*>(kb + (size_t)cur.kslot * kv_dim);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the K tile is there
+    f32x4 vr[4][4];
 #pragma unroll
-      for (int j = 8; j < 16; j++) kr[j] = kp[j];
+    for (int r = 0; r < 4; r++) {
+      const f32x4* vp = reinterpret_cast<const f32x4*>(vb + (size_t)cur.vslot[r] * kv_dim);
+#pragma unroll
+      for (int i = 0; i < 4; i++) vr[r][i] = vp[16 * i];
     }
-
+    __builtin_amdgcn_sched_barrier(0);
     // four independent accumulation chains (one per float4 component)
     f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0, s2 = s0, s3 = s0;
 #pragma unroll
     for (int j = 0; j < 16; j++) {
-      if (j == 8) {  // the first half's K registers are free: V rows load now
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const float4* vp = reinterpret_cast<const float4*>(vb + (size_t)cur.vslot[r] * kv_dim);
-#pragma unroll
-          for (int i = 0; i < 4; i++) vr[r][i] = vp[i];
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      const float4 q4 = qs4[j * 64 + lane];
-      s0 = mfma_f32_4(kr[j].x, q4.x, s0);
-      s1 = mfma_f32_4(kr[j].y, q4.y, s1);
-      s2 = mfma_f32_4(kr[j].z, q4.z, s2);
-      s3 = mfma_f32_4(kr[j].w, q4.w, s3);
+      const float4 k4 = kt[(4 * j + quad) ^ col], q4 = qs4[j * 64 + lane];
+      s0 = mfma_f32_4(k4.x, q4.x, s0);
+      s1 = mfma_f32_4(k4.y, q4.y, s1);
+      s2 = mfma_f32_4(k4.z, q4.z, s2);
+      s3 = mfma_f32_4(k4.w, q4.w, s3);
     }
     const f32x4 s = (s0 + s1) + (s2 + s3);
-    __builtin_amdgcn_sched_barrier(0);  // K registers are free from here on
-    {
-      const float4* kp = reinterpret_cast<const float4*>(kb + (size_t)nxt.kslot * kv_dim);
-#pragma unroll
-      for (int j = 0; j < 8; j++) kr[j] = kp[j];
-    }
-    uint32_t vmask[4];
-#pragma unroll
-    for (int r = 0; r < 4; r++) vmask[r] = cur.vmask[r];
-    cur = nxt;
-    pfm_entries(list, S, tile + 2 * ATT_WAVES, col, quad, nxt);
     float sv[4], mx = -INFINITY;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
       sv[r] = s[r] * a.scale;
-      if ((vmask[r] >> bit) & 1u) mx = fmaxf(mx, sv[r]);
+      if ((cur.vmask[r] >> bit) & 1u) mx = fmaxf(mx, sv[r]);
     }
     mx = swap32_max(swap16_max(mx));
     const float mt = fmaxf(m, mx);
@@ -1260,7 +1261,7 @@ extern "C" __global__ __launch_bounds__(ATT_NT, 2) void gh_pf_attn_m_k(AttnArgs 
     float p[4], ps = 0.f;
 #pragma unroll
     for (int r = 0; r < 4; r++) {
-      p[r] = (vmask[r] >> bit) & 1u ? __expf(sv[r] - mt) : 0.f;
+      p[r] = (cur.vmask[r] >> bit) & 1u ? __expf(sv[r] - mt) : 0.f;
       ps += p[r];
     }
     ps = swap32_add(swap16_add(ps));
@@ -1268,50 +1269,60 @@ extern "C" __global__ __launch_bounds__(ATT_NT, 2) void gh_pf_attn_m_k(AttnArgs 
     m = mt;
 #pragma unroll
     for (int t = 0; t < 16; t++) o[t] *= corr;
+    // The V rows are waited for here, before the next K tile's loads go out:
+    // a later wait would count those too.
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)"
+                 : "+v"(vr[0][0]), "+v"(vr[0][1]), "+v"(vr[0][2]), "+v"(vr[0][3]), "+v"(vr[1][0]),
+                   "+v"(vr[1][1]), "+v"(vr[1][2]), "+v"(vr[1][3])
+                 :
+                 : "memory");
+    asm volatile(""
+                 : "+v"(vr[2][0]), "+v"(vr[2][1]), "+v"(vr[2][2]), "+v"(vr[2][3]), "+v"(vr[3][0]),
+                   "+v"(vr[3][1]), "+v"(vr[3][2]), "+v"(vr[3][3]));
+    cur = nxt;
+    load_k(cur.kslot);
+    __builtin_amdgcn_sched_barrier(0);
+    pfm_entries(list, S, tile + 2 * ATT_WAVES, col, quad, nxt);
 #pragma unroll
     for (int r = 0; r < 4; r++) {
 #pragma unroll
-      for (int t = 0; t < 16; t++) {  // consecutive products into different tiles
-        const float4 v4 = vr[r][t >> 2];
-        const float v = (t & 3) == 0 ? v4.x : (t & 3) == 1 ? v4.y : (t & 3) == 2 ? v4.z : v4.w;
-        o[t] = mfma_f32_4(v, p[r], o[t]);
-      }
+      for (int t = 0; t < 16; t++)  // consecutive products into different tiles
+        o[t] = mfma_f32_4(vr[r][t >> 2][t & 3], p[r], o[t]);
     }
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the last K tile's loads, of no use, are in LDS
 
-  // 3. merge the four waves (wave order) and write the output rows
+  // 3. merge the four waves (wave order) and write the output rows: lane's
+  //    column, wave j the dims 64 j + 16 quad .. + 15
   __syncthreads();  // every wave is done with the query operand (aliased below)
 #pragma unroll
-  for (int t = 0; t < 16; t++) {
-#pragma unroll
-    for (int r = 0; r < 4; r++) wo[(wave * 64 + t * 4 + r) * 64 + lane] = o[t][r];
-  }
+  for (int t = 0; t < 16; t++)
+    smem4[(wave * 16 + t) * 64 + lane] = make_float4(o[t][0], o[t][1], o[t][2], o[t][3]);
   if (quad == 0) {
-    wm[wave][col] = m;
-    wl[wave][col] = l;
+    wm[wave * 16 + col] = m;
+    wl[wave * 16 + col] = l;
   }
   __syncthreads();
-  const uint32_t c = tid >> 4, i = tid & 15;  // output column, dims 16 i .. 16 i + 15
-  const uint32_t t = t0 + c / G, g = c % G;
+  const uint32_t t = t0 + col / G, g = col % G;
   if (t < a.n_tokens) {
     float M = -INFINITY;
-    for (int w = 0; w < ATT_WAVES; w++) M = fmaxf(M, wm[w][c]);
-    float cw[ATT_WAVES], L = 0.f;
-    for (int w = 0; w < ATT_WAVES; w++) {
-      cw[w] = wm[w][c] == -INFINITY ? 0.f : __expf(wm[w][c] - M);
-      L += wl[w][c] * cw[w];
-    }
-    const uint32_t ln = (i >> 2) * 16 + c, r = i & 3;
-    float res[16];
 #pragma unroll
-    for (int d = 0; d < 16; d++) {
-      float O = 0.f;
-      for (int w = 0; w < ATT_WAVES; w++) O += wo[(w * 64 + d * 4 + r) * 64 + ln] * cw[w];
-      res[d] = L > 0.f ? O / L : 0.f;
+    for (int w = 0; w < ATT_WAVES; w++) M = fmaxf(M, wm[w * 16 + col]);
+    float L = 0.f;
+    f32x4 O[4] = {};  // [e]: dims 4 r + e of the wave's 16
+#pragma unroll
+    for (int w = 0; w < ATT_WAVES; w++) {
+      const float mw = wm[w * 16 + col], cw = mw == -INFINITY ? 0.f : __expf(mw - M);
+      L += wl[w * 16 + col] * cw;
+#pragma unroll
+      for (int e = 0; e < 4; e++)
+        O[e] += reinterpret_cast<const f32x4*>(smem4)[(w * 16 + 4 * wave + e) * 64 + lane] * cw;
     }
     float4* dst = reinterpret_cast<float4*>(a.out_rows + (size_t)t * a.out_stride +
-                                            (size_t)(kvh * G + g) * PFM_D + i * 16);
+                                            (size_t)(kvh * G + g) * PFM_D + 64 * wave + 16 * quad);
 #pragma unroll
-    for (int j = 0; j < 4; j++) dst[j] = make_float4(res[4 * j], res[4 * j + 1], res[4 * j + 2], res[4 * j + 3]);
+    for (int r = 0; r < 4; r++)
+      dst[r] = L > 0.f ? make_float4(O[0][r] / L, O[1][r] / L, O[2][r] / L, O[3][r] / L)
+                       : make_float4(0.f, 0.f, 0.f, 0.f);
   }
 }

@@ -611,6 +611,41 @@ def test_model_ring_prefill_staged_head_dim_256(gpu, monkeypatch, T, mfma, split
         p.close()
 
 
+@pytest.mark.parametrize("heads,kv_heads", [(16, 8), (4, 4)])
+@pytest.mark.parametrize("T", [65, 129, 214])
+def test_model_prefill_matrix_attention_tiles(gpu, T, heads, kv_heads):
+    # The matrix-core attention over lists of several 16-slot tiles per
+    # wavefront (its K tiles are loaded one ahead): a whole prompt just past a
+    # tile of each of the four waves, at the edge of the next, and 3 or 4 tiles
+    # per wave with a remainder, after the window's slots were written once by
+    # another prompt; against the per-token path's caches and logits.
+    cfg = gh.model_config(vocab=1024, hidden=512, intermediate=1024, layers=2, heads=heads,
+                          kv_heads=kv_heads, head_dim=256, max_slots=240, full_layers=(1,))
+    m = gh.Model(gpu, cfg, mode=gh.QUANT_Q4, seed=6)
+    p = gh.Model(gpu, cfg, mode=gh.QUANT_Q4, seed=6)
+    try:
+        xs = np.stack([m.embed(i * 53 % cfg.vocab_size) for i in range(2 * T)])
+        for x in (m, p):
+            x.ring_init(4, 230, 6)
+            x.ring_prefill(xs[T:], 0, False)
+            x.ring_init(4, 230, 6)
+        tok = m.ring_prefill(xs[:T], 0, True)
+        for c in range(T):
+            ptok = p.forward_clock(xs[c], c, c == T - 1)
+        logits = m.read(-1, gh.T_LOGITS, np.float32)
+        plog = p.read(-1, gh.T_LOGITS, np.float32)
+        assert_close(logits, plog, what="matrix-core prefill vs per-token logits")
+        assert tok == orc.argmax(logits) and ptok == orc.argmax(plog)
+        for l in range(cfg.num_hidden_layers):
+            for t in (gh.T_K_CACHE, gh.T_V_CACHE):
+                got = m.read(l, t, np.float32).reshape(cfg.max_slots, -1)
+                per = p.read(l, t, np.float32).reshape(cfg.max_slots, -1)
+                assert_close(got[:T], per[:T], what="cache %d/%d" % (l, t))
+    finally:
+        m.close()
+        p.close()
+
+
 def test_model_ring_prefill_staged_chunks_below_ring_size(gpu):
     # A 300-slot cache holds 256 staging rows (min(max_slots, 256)), so a
     # staged batch of 270 tokens runs as chunks of 256 and 14.  Ring of 4
