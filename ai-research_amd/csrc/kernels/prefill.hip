@@ -6,8 +6,7 @@
 // src/gpu/model_dispatch.zig:144).  Here the T prompt tokens of a layer go
 // through each projection as one dense contraction
 //     C[T][N] = A[T][K] . deq(W)[N][K]^T
-// on the matrix cores (v_mfma_f32_32x32x16_f16), keeping the decode path's
-// accuracy:
+// on the matrix cores, keeping the decode path's accuracy:
 //  * weights enter exactly: the MFMA B operand is the integer n - 8 (Q4) or
 //    q (Q8), exact in fp16, and each 32-block's f32 scale d is applied to the
 //    block's fp32 partial sum (acc += d * block_sum), as the GEMV does;
@@ -20,7 +19,13 @@
 //    (exact: a power of two);
 //  * accumulation is fp32.
 //
-// Tiling: a workgroup of 256 threads (2 x 2 wavefronts) owns a BM x BN tile
+// Three forms, chosen by the host: the weight-streaming GEMM for short batches,
+// the wide tile for longer ones (both described at their kernels below), and
+// the tiles that follow for what those do not take: K that is no multiple of
+// 128, or weights that are not 16-byte aligned.
+//
+// Tiling (v_mfma_f32_32x32x16_f16): a workgroup of 256 threads (2 x 2
+// wavefronts) owns a BM x BN tile
 // of C; each wavefront a (BM/2) x (BN/2) sub-tile of 32 x 32 MFMA blocks (the
 // _w8 forms of the 128-row tiles: 512 threads, 4 x 2 wavefronts of
 // (BM/4) x (BN/2), so a CU's two tiles run four waves per SIMD).  K

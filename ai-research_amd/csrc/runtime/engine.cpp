@@ -619,13 +619,14 @@ gh_status launch_prefill_gemm_split(gh_context* ctx, gh_quant_mode mode, const v
     return launch_prefill_stream(ctx, mode, W0, W1, Ax, rs, C, T, N, K, planes, nplanes, false);
   // Longer batches take the wide tile, 1.02-1.75x the speed of the tiles below
   // wherever both were measured (wide_shape).  Those stay for K that is no
-  // multiple of 128 and for weights that are not 16-byte aligned.
+  // multiple of 128 and for weights that are not 16-byte aligned; their rules'
+  // figures are of the 12B products, which they served before the wide tile.
   if (wide_ok(K, W0, W1))
     return launch_prefill_wide(ctx, mode, W0, W1, Ax, rs, C, T, N, K, planes, nplanes);
   // A product without planes of 256k + 1..127 tokens (a 288-token gate+up:
   // 720 tiles, the last 240 three-quarters padding) runs as two products: the
-  // multiple of 256 on the tiles, the rest as its own product (the
-  // weight-streaming GEMM up to 48 tokens, tiles above).  Prompts of 272 /
+  // multiple of 256 on the tiles, the rest as its own product (the streamed
+  // GEMM up to 48 tokens and tiles above, when measured).  Prompts of 272 /
   // 288 / 300 / 320 / 352 tokens: 26.8 / 26.8 / 26.9 / 27.3 / 27.6 -> 23.3 /
   // 23.9 / 24.6 / 25.1 / 26.6 ms (GH_PF_REST_MAX=n: at most n tokens).
   const uint32_t rest = T % 256;

@@ -1618,10 +1618,9 @@ gh_status prefill_forward(gh_model* m, uint32_t T, bool want_logits,
                                       m->pf_m, T, H, I, last ? nullptr : &m_planes,
                                       last ? nullptr : &m_nz)) != GH_OK)
       return st;
-    // Many planes (the streamed down projection of a short prompt: 30) are
-    // summed over all CUs first: the norm reads its token's planes from one
-    // CU each, and at 16 tokens took 14.4 us with 30 planes against 5.2 us
-    // with one.
+    // Many planes (the streamed down projection of 16 tokens: 15) are summed
+    // over all CUs first: the norm reads its token's planes from one CU each,
+    // and at 16 tokens took 14.4 us with 30 planes against 5.2 us with one.
     if (m_nz > 8) {
       if ((st = gh::launch_prefill_plane_sum(ctx, m_planes, m->pf_m, T, H, m_nz)) != GH_OK)
         return st;
