@@ -107,13 +107,16 @@ struct gh_model {
   // gh_qgate_k launch instead of gating in their QKV stream's prologue
   bool qgate_kernel = false;
   // A prompt of at most this many tokens runs token by token through the
-  // decode graphs: a single one.  At the 12B shape in Q4 it takes 2.66 ms that
-  // way, and 3 tokens in one batched call (whose projections stream the
-  // weights once for all tokens) 4.15; two tokens in 2 / 12 such layers 318 /
-  // 1354 us token by token, 241 / 1051 us in one call.  Set at init;
-  // GH_PF_SEQ_MAX (read at init) overrides it, and 0 sends every prompt to the
-  // batched kernels.
-  uint32_t seq_prefill_max = 1;
+  // decode graphs.  One token: 2.66 ms at the 12B shape in Q4, where 3 tokens
+  // in one batched call (whose projections stream the weights once for all
+  // tokens) take 4.15.  Two Q4 tokens: the graphs multiply in f32 where the
+  // batched call's activations enter as two fp16 halves (22 bits), so they stay
+  // there although one call is faster (2 / 12 such layers 318 / 1354 us token
+  // by token, 241 / 1051 us in one call).  Q8 and bf16 decode steps take 3.7 and
+  // 5.0 ms, and there only a single token runs that way.  Set at init from the
+  // weight mode; GH_PF_SEQ_MAX (read at init) overrides it, and 0 sends every
+  // prompt to the batched kernels.
+  uint32_t seq_prefill_max = 2;
   // layer gating (quiescence): layers >= num_layers / 3 are gated when on
   bool q_on = false;
   float q_thr = 0.f;
@@ -604,9 +607,7 @@ gh_status finish_init(gh_model* m, gh_model** out) {
   m->eager = eager && eager[0] == '1';
   const char* qk = getenv("GH_QGATE_KERNEL");
   m->qgate_kernel = qk && qk[0] == '1';
-  // 2 where the prefill GEMMs do not take the model's widest product
-  m->seq_prefill_max =
-      m->mode == GH_QUANT_Q4 && std::max(m->max_q, m->cfg.intermediate_size) > 16384u ? 2u : 1u;
+  m->seq_prefill_max = m->mode == GH_QUANT_Q4 ? 2u : 1u;
   if (const char* sq = getenv("GH_PF_SEQ_MAX")) m->seq_prefill_max = (uint32_t)strtoul(sq, nullptr, 10);
   gh_status st = reset_gates(m);
   if (st == GH_OK) st = record_graphs(m);

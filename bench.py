@@ -599,8 +599,8 @@ def bench_decode(ctx, n_prompt=512, n_decode=128, cpu=False):
             times.append(time.perf_counter() - t0)
             c += T
         wrapped[str(T)] = round(sorted(times)[1] * 1e3, 2)
-    # short first-turn prompts (clocks from 0, after the run): a single token
-    # goes through the decode graph, longer ones to the batched
+    # short first-turn prompts (clocks from 0, after the run): 1-2 tokens go
+    # token by token through the decode graphs, longer ones to the batched
     # kernels (the weight-streaming GEMMs up to 48 tokens); median of 3 calls
     # each
     short = {}

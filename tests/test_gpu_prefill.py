@@ -345,9 +345,10 @@ def test_model_prefill_matches_sequential_oracle(gpu, monkeypatch, mode, T, dup,
     # not a multiple of 4 leaves a partial token group in the grouped
     # attention; dup names one slot twice in the last token's list (counted
     # twice, as the reference's loop over the list does), which keeps the
-    # batch on the per-token attention kernel.  A single token runs through
-    # the decode graphs unless GH_PF_SEQ_MAX=0 keeps it on the batched kernels
-    # (GH_PF_SEQ_MAX=3 sends 3 tokens token by token)
+    # batch on the per-token attention kernel.  Batches of 1-2 tokens (Q4;
+    # 1 token with Q8 weights) run token by token unless GH_PF_SEQ_MAX=0 keeps
+    # them on the batched kernels (GH_PF_SEQ_MAX=3 sends 3 tokens token by
+    # token)
     if seq_max is not None:
         monkeypatch.setenv("GH_PF_SEQ_MAX", seq_max)
     cfg = tiny_cfg()
@@ -380,6 +381,27 @@ def test_model_prefill_matches_sequential_oracle(gpu, monkeypatch, mode, T, dup,
             assert_close(m.read(-1, gh.T_LOGITS, np.float32), rlog, what="decode after prefill")
     finally:
         m.close()
+
+
+def test_two_q4_tokens_are_the_decode_graphs(gpu):
+    # two Q4 tokens in one call are the two per-token calls to the bit: the
+    # graphs multiply in f32, where a batched call's activations enter the
+    # matrix cores as two fp16 halves
+    cfg = tiny_cfg()
+    a, b = (gh.Model(gpu, cfg, mode=gh.QUANT_Q4, seed=12) for _ in range(2))
+    try:
+        ring = gh.Ring(cfg.num_hidden_layers, 4, 16, 4)
+        xs = np.stack([a.embed(t) for t in (3, 700)])
+        slots, actives = ring_lists(ring, range(2))
+        tok = a.prefill(xs, np.arange(2), slots, actives, True)
+        b.forward(xs[0], 0, slots[0], actives[0], False)
+        assert tok == b.forward(xs[1], 1, slots[1], actives[1], True)
+        for layer, t in [(-1, gh.T_LOGITS)] + [(l, t) for l in range(cfg.num_hidden_layers)
+                                               for t in (gh.T_K_CACHE, gh.T_V_CACHE)]:
+            assert np.array_equal(a.read(layer, t, np.uint32), b.read(layer, t, np.uint32)), (layer, t)
+    finally:
+        a.close()
+        b.close()
 
 
 def test_model_prefill_norm_forms_bit_identical(gpu, monkeypatch):
