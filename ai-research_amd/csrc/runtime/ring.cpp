@@ -84,42 +84,21 @@ uint32_t gh_ring_active_slots(const gh_ring* r, uint32_t layer, uint64_t clock, 
     if (n < cap) out[n] = (uint32_t)s;
     n++;
   };
-  // Slots [from, to) that are active with a clock in [minc, clock].  Eight
-  // inactive slots (a window that is still filling, unused recall slots) cost
-  // one load, and a slot with room in `out` costs no branch: a prompt asks for
-  // every token's list, at 512 tokens over 640 slots 330k of them.
-  const uint8_t* flag = &r->active[base];
-  const uint64_t* when = &r->clocks[base];
-  auto live = [&](size_t from, size_t to, uint64_t minc) {
-    for (size_t s = from; s < to;) {
-      const size_t end = to - s < 8 ? to : s + 8;
-      if (end - s == 8) {
-        uint64_t any;
-        memcpy(&any, flag + s, 8);
-        if (any == 0) {
-          s = end;
-          continue;
-        }
-      }
-      if (cap >= 8 && n <= cap - 8) {
-        for (; s < end; s++) {
-          out[n] = (uint32_t)s;
-          n += (uint32_t)(flag[s] != 0) & (uint32_t)(when[s] >= minc) & (uint32_t)(when[s] <= clock);
-        }
-      } else {
-        for (; s < end; s++)
-          if (flag[s] && when[s] >= minc && when[s] <= clock) push(s);
-      }
-    }
-  };
   const size_t alim = clock + 1 < r->num_anchors ? (size_t)clock + 1 : r->num_anchors;
   for (size_t s = 0; s < alim; s++)
     if (r->active[base + s]) push(s);
   if (clock >= r->num_anchors) {
     const uint64_t minc = clock >= r->window_size ? clock - r->window_size + 1 : r->num_anchors;
-    live(r->num_anchors, r->recall_start(), minc);
+    for (size_t s = r->num_anchors; s < r->recall_start(); s++) {
+      if (!r->active[base + s]) continue;
+      const uint64_t c = r->clocks[base + s];
+      if (c >= minc && c <= clock) push(s);
+    }
   }
-  live(r->recall_start(), r->total_slots, 0);
+  for (size_t s = r->recall_start(); s < r->total_slots; s++) {
+    if (!r->active[base + s]) continue;
+    if (r->clocks[base + s] <= clock) push(s);
+  }
   return n;
 }
 

@@ -75,3 +75,22 @@ def test_ring_lists_by_room():
                     assert n == len(want)
                     assert np.array_equal(out[:min(n, cap)], want[:cap])
                     assert (out[cap:] == 0xFFFFFFFF).all()
+
+
+def test_ring_lists_leave_the_room_behind_them():
+    """Room past the list's end keeps what it held: a host may pack lists one
+    behind another, or keep words of its own there."""
+    rng = np.random.default_rng(8)
+    for A, W, R in [(32, 512, 96), (3, 13, 5), (0, 24, 0), (9, 8, 1), (2, 16, 8)]:
+        g = gh.Ring(1, A, W, R)
+        for c in range(2 * W):
+            if rng.random() < 0.7:
+                g.activate_slot(0, c)
+            if R and rng.random() < 0.2:
+                g.activate_recall(0, int(rng.integers(0, R)), int(rng.integers(0, 2 * W)))
+            q = int(rng.integers(0, c + 2))
+            want = g.active_slots(0, q)
+            out = np.full(g.total_slots + 16, 0xFFFFFFFF, np.uint32)
+            n = gh.lib().gh_ring_active_slots(g.h, 0, q, gh._ptr(out), len(out))
+            assert n == len(want) and np.array_equal(out[:n], want)
+            assert (out[n:] == 0xFFFFFFFF).all()
