@@ -157,6 +157,8 @@ gh_status prefill_forward(gh_model* m, uint32_t T, bool want_logits,
 gh_status prefill_batch(gh_model* m, const float* x, bool x_up, uint32_t T, const uint64_t* clocks,
                         const uint32_t* slot_idx, const uint32_t* active, uint32_t active_stride,
                         const uint32_t* n_active, int want_logits, uint32_t* out_token);
+gh_status ring_prefill(gh_model* m, const float* x, uint32_t T, uint64_t first_clock,
+                       int want_logits, uint32_t* out_token);
 }  // namespace
 
 gh_model::~gh_model() {
@@ -635,8 +637,9 @@ gh_status reset_gates(gh_model* m) {
   return st;
 }
 
-// Sends the host mirror's layer-0 ring state to the device arrays the ring
-// kernel reads.
+using RingPtr = std::unique_ptr<gh_ring, void (*)(gh_ring*)>;
+RingPtr ring_copy(const gh_ring* r) { return RingPtr(gh::ring_clone(r), gh_ring_destroy); }
+
 // Queues the copy of ring `r`'s layer 0 state; `st` holds it until the copy
 // is done.
 hipError_t ring_queue(gh_model* m, const gh_ring* r, std::vector<uint32_t>* st) {
@@ -651,12 +654,40 @@ hipError_t ring_queue(gh_model* m, const gh_ring* r, std::vector<uint32_t>* st) 
   return e;
 }
 
+// Sends the host mirror's layer-0 ring state to the device arrays the ring
+// kernel reads.
 gh_status ring_upload(gh_model* m) {
   std::vector<uint32_t> st;
   hipError_t e = ring_queue(m, m->ring, &st);
   const hipError_t es = hipStreamSynchronize(m->ctx->stream);
   if (e == hipSuccess) e = es;
   return e == hipSuccess ? GH_OK : hip_fail(e, "ring state copy");
+}
+
+// Waits for the stream when it goes out of scope: declared behind the host
+// memory that queued copies read, it keeps that alive on every way out.
+struct StreamWait {
+  hipStream_t stream;
+  ~StreamWait() { done(); }
+  hipError_t done() {
+    const hipError_t e = stream ? hipStreamSynchronize(stream) : hipSuccess;
+    stream = nullptr;
+    return e;
+  }
+};
+
+// An entry point's body: running out of host memory is a status there.
+template <class F>
+gh_status no_throw(const char* who, F body) {
+  try {
+    return body();
+  } catch (const std::bad_alloc&) {
+    try {
+      return fail(GH_ERR_ALLOC, std::string(who) + ": out of host memory");
+    } catch (const std::bad_alloc&) {
+      return GH_ERR_ALLOC;
+    }
+  }
 }
 
 gh_status rerecord(gh_model* m) {
@@ -1009,48 +1040,8 @@ gh_status gh_model_ring_prefill(gh_model* m, const float* x, uint32_t T, uint64_
   if (!m->ring) return fail(GH_ERR_INVALID, "gh_model_ring_prefill: gh_model_ring_init first");
   if (T == 0 || first_clock + T - 1 > 0xFFFFFFFFull)
     return fail(GH_ERR_INVALID, "gh_model_ring_prefill: T is zero or a clock exceeds 2^32");
-  const uint32_t total = gh_ring_total_slots(m->ring);
-  std::vector<uint64_t> clocks(T);
-  std::vector<uint32_t> slots(T), n(T);
-  std::unique_ptr<uint32_t[]> lists(new (std::nothrow) uint32_t[(size_t)T * total]);
-  if (!lists) return fail(GH_ERR_ALLOC, "gh_model_ring_prefill: active lists");
-  // the lists as the per-token calls would see them: slot activations of the
-  // earlier tokens of the batch included, later ones not; a failed call
-  // leaves the ring as it was
-  gh_ring* r = gh::ring_clone(m->ring);
-  if (!r) return fail(GH_ERR_ALLOC, "gh_model_ring_prefill: ring copy");
-  // the call below advances m->ring as its tokens or chunks finish: keep
-  // the state from before the call to put back on failure
-  gh_ring* before = gh::ring_clone(m->ring);
-  if (!before) {
-    gh_ring_destroy(r);
-    return fail(GH_ERR_ALLOC, "gh_model_ring_prefill: ring copy");
-  }
-  // A batch whose buffers are there starts its x on the way before its lists
-  // are built: at 512 tokens the copy call takes 150 us, the copy 230, and
-  // the lists and their checks 160.  A batch that runs in parts copies its
-  // rows again, to the same buffer and behind this copy.
-  const bool x_up = T > m->seq_prefill_max && !(m->q_on && want_logits) && m->pf_arena &&
-                    m->pf_cap >= T && m->pf_stride >= total && m->cfg.hidden_size <= 8192 &&
-                    hipMemcpyAsync(m->pf_x, x, (size_t)T * m->cfg.hidden_size * 4,
-                                   hipMemcpyHostToDevice, m->ctx->stream) == hipSuccess;
-  for (uint32_t t = 0; t < T; t++) {
-    clocks[t] = first_clock + t;
-    slots[t] = gh_ring_activate_slot(r, 0, clocks[t]);
-    n[t] = gh_ring_active_slots(r, 0, clocks[t], lists.get() + (size_t)t * total, total);
-  }
-  gh_status st = prefill_batch(m, x, x_up, T, clocks.data(), slots.data(), lists.get(), total,
-                               n.data(), want_logits, out_token);
-  gh_ring_destroy(r);
-  if (st == GH_OK) {  // m->ring and the device's copy have taken the batch's activations
-    gh_ring_destroy(before);
-    return GH_OK;
-  }
-  const std::string why = gh_last_error();
-  gh_ring_destroy(m->ring);
-  m->ring = before;
-  ring_upload(m);  // also waits for the copy of x
-  return fail(st, why);
+  return no_throw("gh_model_ring_prefill",
+                  [&] { return ring_prefill(m, x, T, first_clock, want_logits, out_token); });
 }
 
 gh_status gh_model_set_quiescence(gh_model* m, float threshold) {
@@ -1079,13 +1070,57 @@ gh_status gh_model_prefill(gh_model* m, const float* x, uint32_t T, const uint64
                            const uint32_t* slot_idx, const uint32_t* active,
                            uint32_t active_stride, const uint32_t* n_active, int want_logits,
                            uint32_t* out_token) {
-  return prefill_batch(m, x, false, T, clocks, slot_idx, active, active_stride, n_active,
-                       want_logits, out_token);
+  return no_throw("gh_model_prefill", [&] {
+    return prefill_batch(m, x, false, T, clocks, slot_idx, active, active_stride, n_active,
+                         want_logits, out_token);
+  });
 }
 
 }  // extern "C"
 
 namespace {
+
+gh_status ring_prefill(gh_model* m, const float* x, uint32_t T, uint64_t first_clock,
+                       int want_logits, uint32_t* out_token) {
+  const uint32_t total = gh_ring_total_slots(m->ring);
+  // the lists as the per-token calls would see them: slot activations of the
+  // earlier tokens of the batch included, later ones not; a failed call
+  // leaves the ring as it was: prefill_batch advances m->ring as its tokens or
+  // chunks finish, so the state from before the call is kept to put back
+  RingPtr r = ring_copy(m->ring), before = ring_copy(m->ring);
+  std::vector<uint32_t> words(2 * (size_t)m->cfg.max_slots);
+  const gh_status st = no_throw("gh_model_ring_prefill", [&] {
+    std::vector<uint64_t> clocks(T);
+    std::vector<uint32_t> slots(T), n(T);
+    const std::unique_ptr<uint32_t[]> lists(new uint32_t[(size_t)T * total]);
+    // A batch whose buffers are there starts its x on the way before its lists
+    // are built: at 512 tokens the copy call takes 150 us, the copy 230, and
+    // the lists and their checks 160.  A batch that runs in parts copies its
+    // rows again, to the same buffer and behind this copy.
+    StreamWait x_read{nullptr};
+    const bool x_up = T > m->seq_prefill_max && !(m->q_on && want_logits) && m->pf_arena &&
+                      m->pf_cap >= T && m->pf_stride >= total && m->cfg.hidden_size <= 8192 &&
+                      hipMemcpyAsync(m->pf_x, x, (size_t)T * m->cfg.hidden_size * 4,
+                                     hipMemcpyHostToDevice, m->ctx->stream) == hipSuccess;
+    if (x_up) x_read.stream = m->ctx->stream;
+    for (uint32_t t = 0; t < T; t++) {
+      clocks[t] = first_clock + t;
+      slots[t] = gh_ring_activate_slot(r.get(), 0, clocks[t]);
+      n[t] = gh_ring_active_slots(r.get(), 0, clocks[t], lists.get() + (size_t)t * total, total);
+    }
+    const gh_status bs = prefill_batch(m, x, x_up, T, clocks.data(), slots.data(), lists.get(),
+                                       total, n.data(), want_logits, out_token);
+    if (bs == GH_OK) x_read.stream = nullptr;  // the batch has waited for it
+    return bs;
+  });
+  if (st != GH_OK) {  // (with `words` there, and the error's message left as it is)
+    gh_ring_destroy(m->ring);
+    m->ring = before.release();
+    ring_queue(m, m->ring, &words);
+    hipStreamSynchronize(m->ctx->stream);
+  }
+  return st;  // done: m->ring and the device's copy have taken the batch's activations
+}
 
 // gh_model_prefill; with x_up the copy of x to m->pf_x is already queued.
 gh_status prefill_batch(gh_model* m, const float* x, bool x_up, uint32_t T, const uint64_t* clocks,
@@ -1204,6 +1239,13 @@ gh_status prefill_batch(gh_model* m, const float* x, bool x_up, uint32_t T, cons
     meta[T + t] = conflict ? nslot + t : slot_idx[t];
     meta[2 * T + t] = n_active[t];
   }
+  // What the queued copies read, and the ring's next state, with the wait that
+  // every way out below takes before any of it is freed.
+  std::vector<uint32_t> act, ucount, ring_words(m->ring ? 2 * (size_t)nslot : 0);
+  std::unique_ptr<uint32_t[]> uni;
+  std::vector<uint8_t> table;
+  RingPtr ring = ring_copy(m->ring);
+  StreamWait wait{s};
   hipError_t e = hipSuccess;
   if (!x_up) e = hipMemcpyAsync(m->pf_x, x, (size_t)T * c.hidden_size * 4, hipMemcpyHostToDevice, s);
   if (e == hipSuccess) e = hipMemcpyAsync(m->pf_meta, meta.data(), meta.size() * 4, hipMemcpyHostToDevice, s);
@@ -1241,10 +1283,7 @@ gh_status prefill_batch(gh_model* m, const float* x, bool x_up, uint32_t T, cons
   }
   // The attention's lists, built and copied once layer 0's projection is
   // queued: no earlier kernel reads them, so the host's pass over them (at 512
-  // tokens some 130k entries) runs while the GPU works.  They live to the end
-  // of this call, as the copies may still read them.
-  std::vector<uint32_t> act, ucount;
-  std::unique_ptr<uint32_t[]> uni;
+  // tokens some 130k entries) runs while the GPU works.
   m->pf_gkind = 0;
   auto attention_lists = [&]() -> gh_status {
     hipError_t e = hipSuccess;
@@ -1253,8 +1292,7 @@ gh_status prefill_batch(gh_model* m, const float* x, bool x_up, uint32_t T, cons
       const uint32_t groups = (T + gtok - 1) / gtok;
       const uint32_t ustride = std::min(gtok * m->pf_stride, nrows);
       const size_t words = (size_t)groups * ustride * 2;
-      uni.reset(new (std::nothrow) uint32_t[words]);  // entries past a group's count are not read
-      if (!uni) return fail(GH_ERR_ALLOC, "gh_model_prefill: union lists");
+      uni.reset(new uint32_t[words]);  // entries past a group's count are not read
       ucount.assign(groups, 0u);
       std::vector<uint32_t> stamp(nrows, 0u), pos(nrows);
       for (uint32_t g = 0; g < groups && ok; g++) {
@@ -1298,7 +1336,6 @@ gh_status prefill_batch(gh_model* m, const float* x, bool x_up, uint32_t T, cons
     }
     return e == hipSuccess ? GH_OK : hip_fail(e, "gh_model_prefill: list copies");
   };
-  std::vector<uint8_t> table;
   if (conflict) {  // offsets and row words of every cache, then the pairs
     const size_t nc = 2 * m->layers.size();
     table.resize(nc * 12 + pairs.size() * 4);
@@ -1323,10 +1360,7 @@ gh_status prefill_batch(gh_model* m, const float* x, bool x_up, uint32_t T, cons
     m->pf_trace_cap = T;
   }
   if (m->trace_on) m->pf_trace_T = T;
-  if ((st = prefill_forward(m, T, want_logits != 0, attention_lists)) != GH_OK) {
-    hipStreamSynchronize(s);  // the copies read this call's vectors
-    return st;
-  }
+  if ((st = prefill_forward(m, T, want_logits != 0, attention_lists)) != GH_OK) return st;
   if (conflict) {
     const size_t nc = 2 * m->layers.size();
     uint8_t* base = m->arena;
@@ -1344,13 +1378,11 @@ gh_status prefill_batch(gh_model* m, const float* x, bool x_up, uint32_t T, cons
   }
   // the ring's new state goes up behind the layers; the host's takes it once
   // they are done
-  std::unique_ptr<gh_ring, void (*)(gh_ring*)> ring(gh::ring_clone(m->ring), gh_ring_destroy);
-  std::vector<uint32_t> ring_words;
   if (ring) {
     for (uint32_t t = 0; t < T; t++) gh_ring_activate_slot(ring.get(), 0, clocks[t]);
     e = ring_queue(m, ring.get(), &ring_words);
   }
-  const hipError_t es = hipStreamSynchronize(s);
+  const hipError_t es = wait.done();
   if (e == hipSuccess) e = es;
   if (e != hipSuccess) return hip_fail(e, "gh_model_prefill");
   m->hidden_final = want_logits ? m->x1 : kNone;
