@@ -111,6 +111,7 @@ extern "C" __global__ __launch_bounds__(64) void gh_qkv_rope_k(
 // split-K decode attention
 // ---------------------------------------------------------------------------
 #include "../common/attn_args.h"
+#include "../common/load_lds.h"
 
 // Full-wavefront sum with every lane receiving the same, bit-identical total:
 // DPP butterflies inside each row of 16 lanes (xor 1, xor 2, half-row
@@ -1161,13 +1162,6 @@ __device__ __forceinline__ void pfm_entries(const uint32_t* list, uint32_t S, ui
   }
 }
 
-// 16 bytes per lane from base + off to LDS byte lds + 16 * lane.
-__device__ __forceinline__ void pfm_load_lds16(uint32_t off, const void* base, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off),
-               "s"(base), "s"(lds)
-               : "memory");
-}
-
 extern "C" __global__ __launch_bounds__(ATT_NT, 2) void gh_pf_attn_m_k(AttnArgs a) {
   // a K tile per wave and the query operand (16 steps x 64 lanes of float4);
   // after the loop the waves' o registers and (m, l) take their places
@@ -1204,7 +1198,7 @@ extern "C" __global__ __launch_bounds__(ATT_NT, 2) void gh_pf_attn_m_k(AttnArgs 
 #pragma unroll
     for (int j = 0; j < 16; j++) {
       const uint32_t slot = __builtin_amdgcn_readlane(kslot, j);
-      pfm_load_lds16(16 * (lane ^ j), kb + (size_t)slot * kv_dim, k_lds + 1024 * j);
+      load_lds16(16 * (lane ^ j), kb + (size_t)slot * kv_dim, k_lds + 1024 * j);
     }
   };
   load_k(cur.kslot);

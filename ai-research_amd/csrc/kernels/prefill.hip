@@ -42,6 +42,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "../common/load_lds.h"
+
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
@@ -468,17 +470,6 @@ GH_GEMM_PAIR_W8(gh_pf_gateup_q4_m128_n64, Q4W, 128, 64, 1, true, _s_w8)
 // ---------------------------------------------------------------------------
 #define PF_WIDE_NT 512
 
-// 16 bytes per lane from src to LDS byte lds + 16 * lane.
-__device__ __forceinline__ void load_lds16(const void* src, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src),
-               "s"(lds)
-               : "memory");
-}
-__device__ __forceinline__ void load_lds16(uint32_t off, const void* base, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off),
-               "s"(base), "s"(lds)
-               : "memory");
-}
 template <int N>
 __device__ __forceinline__ void wait_loads_barrier() {
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
