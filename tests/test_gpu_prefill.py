@@ -281,6 +281,30 @@ def test_prefill_stream_cuts(gpu, monkeypatch, mode, T, N, K, cut):
         assert_close(out[:T].view(np.float32), ref, rtol=rtol, what="streamed, cut %s" % cut)
 
 
+# The f32 sums over K: runs of 16 blocks added up by themselves.  Whole activations
+# (their lo halves are zero) and whole weights make every block's sum exact, so
+# what differs from the fp64 product is the rounding of the additions alone.  One
+# of them is off by 2^-23 / sqrt(12) of its binade, 2.5e-8 of its result in the
+# rms; a chain of n like terms by 2.5e-8 sqrt(n / 2) of its sum; runs, their sums
+# and the planes make n + ... of 16, blocks / 16 / planes and planes.  A quarter
+# above that fails a chain over all of K (1.6e-7 to 2.0e-7 here).
+@pytest.mark.parametrize("mode", [gh.QUANT_Q4, gh.QUANT_Q8])
+@pytest.mark.parametrize("T,K,env,planes", [
+    (16, 4864, ("GH_PF_STREAM", "76,1,8"), 2), (5, 4864, ("GH_PF_STREAM", "76,1,8"), 2),
+    (30, 2304, ("GH_PF_STREAM", "36,2,8"), 2), (45, 2048, ("GH_PF_STREAM", "24,1,8"), 3)])
+def test_prefill_sums_in_runs(gpu, monkeypatch, mode, T, K, env, planes):
+    monkeypatch.setenv(*env)
+    N = 512
+    wq, deq = quantized(N, K, mode, 397)
+    a = np.random.default_rng(398).integers(-8, 9, (T, K)).astype(np.float32)
+    W, A, C = gpu.upload(wq), gpu.upload(a), gpu.alloc(T * N * 4)
+    gpu.prefill_gemm(mode, W, A, C, T, N, K)
+    ref = a.astype(np.float64) @ deq.T
+    err = np.linalg.norm(C.read(np.float32, T * N).reshape(T, N) - ref) / np.linalg.norm(ref)
+    n = 16 + K / 32 / 16 / planes + planes
+    assert err <= 1.25 * 2.53e-8 * np.sqrt(n / 2), (err, n)
+
+
 @pytest.mark.parametrize("N", [320, 203])
 @pytest.mark.parametrize("pair", [False, True])
 @pytest.mark.parametrize("split", ["1", "3", "200"])
