@@ -458,15 +458,27 @@ GH_GEMM_PAIR_W8(gh_pf_gateup_q4_m128_n64, Q4W, 128, 64, 1, true, _s_w8)
 //    of a row) at a time, and each wavefront unpacks the words of its rows as
 //    it reads them: a quarter (Q4) of the LDS bytes of fp16 weights;
 //  * one barrier per step, ahead of the last 16 rows, whose MFMAs then cover
-//    the next step's first LDS reads; two to four steps of A in flight.
+//    the next step's first LDS reads; two to four steps of A in flight (one for
+//    the largest Q8 tile, whose weights leave LDS for two stages).
 // The waits are written out (vmcnt counts the loads issued since), because the
 // compiler would wait for every load to LDS before any LDS read.
 //
-// Measured, 12B gate/up of 512 tokens (activation split included): Q4 309 ->
-// 207 us (1170 TFLOP/s executed), Q8 315 -> 218, bf16 338 -> 187; without its
-// loads the Q4 form takes 200 of 225 us, without the LDS reads of A as well
-// 176.  The gate/up of 128 tokens (TM 2, BR 128, which keeps K unsplit) 91 ->
-// 70 us, of 64 tokens 64 -> 53 us.
+// Sums: an fp32 chain over all of an unsplit K is off by more than the split
+// tiles' shorter ones, so runs of blocks (16 for long K) are chains of their own
+// whose sums are added up in second registers.  The tiles of 192 and 256 tokens
+// by 256 rows have registers for only 2 of 6 and 1 of 8 of their 16-row blocks
+// (bf16: for none, but its 16-bit activations are 10 times further off); they
+// take the products that were unsplit before.  Against 64 bits, tile GEMM / one
+// chain / runs, Q4: gate/up 2 x 15360 x 3840 of 64, 128 and 333 tokens 2.05 / 3.09
+// / 1.72e-7, 2.35 / 3.10 / 1.72e-7 and 2.95 / 3.11 / 2.66e-7, down 3840 x 15360 of
+// 128 tokens 1.43 / 1.65 / 1.17e-7.  It takes 2.4% in the mean of 165 products.
+//
+// Measured, 12B gate/up of 512 tokens, tile GEMM -> this (the whole call, its
+// activation split included): Q4 275 -> 206 us (1170 TFLOP/s executed), Q8 295 ->
+// 217, bf16 272 -> 187.  Within a whole prompt's trace the Q4 kernel takes 224 us,
+// at a lower clock.  Timing-only copies took 11% less without the loads, 22%
+// without the LDS reads of A as well.  The gate/up of 128 tokens (TM 2, BR 128,
+// which keeps K unsplit) 89 -> 74 us, of 64 tokens 62 -> 53 us.
 // ---------------------------------------------------------------------------
 #define PF_WIDE_NT 512
 
@@ -657,6 +669,15 @@ __device__ __forceinline__ void wide_tile(const _Float16* __restrict__ Ax,
   for (int i = 0; i < MT; i++)
 #pragma unroll
     for (int c = 0; c < NT; c++) acc[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // the runs' sums: of as many of the 16-row blocks as registers are left for
+  constexpr int MR = TM <= 2 || BR == 128 ? MT : F::kBf16 ? 0 : TM == 3 ? 2 : 1;
+  f32x4 runs[MR > 0 ? MR : 1][NT];
+#pragma unroll
+  for (int i = 0; i < MR; i++)
+#pragma unroll
+    for (int c = 0; c < NT; c++) runs[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const uint32_t nrun = q_end - q_begin;
+  const uint32_t run = nrun > 16 ? 4 : nrun > 4 ? 2 : 1;  // groups of a run
 
   uint32_t step = 4 * q_begin;
   // first loads: the first groups of W and the first NS - 1 steps of A
@@ -783,11 +804,27 @@ __device__ __forceinline__ void wide_tile(const _Float16* __restrict__ Ax,
       st = sn;
     }
     bq = bq + 1 == (uint32_t)NG ? 0 : bq + 1;
+    const bool end = ((q + 1 - q_begin) & (run - 1)) == 0;
+    if (MR < MT || end) {  // (the larger tiles: selects, a branch would spill)
+#pragma unroll
+      for (int i = 0; i < MR; i++)
+#pragma unroll
+        for (int c = 0; c < NT; c++)
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            runs[i][c][e] += end ? acc[i][c][e] : 0.f;
+            acc[i][c][e] = end ? 0.f : acc[i][c][e];
+          }
+    }
   }
   if constexpr (!F::kBf16) {
 #pragma unroll
     for (int e = 0; e < 4 * NT; e++) acc[MT - 1][e / 4][e % 4] += dp[e / 4] * t[1][e / 4][e % 4];
   }
+#pragma unroll
+  for (int i = 0; i < MR; i++)
+#pragma unroll
+    for (int c = 0; c < NT; c++) acc[i][c] += runs[i][c];
   // no load to LDS may outlive the workgroup
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 
@@ -1010,11 +1047,11 @@ extern "C" __global__ __launch_bounds__(PF_NT) void gh_pf_splitk_k(const float* 
 // 13.5 -> 8.1 / 9.5 / 12.4, down 22 / 23 / 30 -> 16.7 / 19.6 / 25.2; Q8 gate/up of 16
 // and 32 tokens 51 / 70 -> 38 / 48.
 //
-// Sums: a set's blocks are one fp32 chain, the sets' sums of a slice a second and
+// Sums: half a set's blocks are one fp32 chain, these sums of a slice a second and
 // the planes a third, so that wide slices cost no precision: against 64 bits the
-// gate/up of 16 tokens (two slices of 60 blocks) is off by 1.66e-7, 2.34e-7 with
-// one chain per slice, 1.71e-7 in slices of 16 blocks.  It takes no measurable
-// time (216 products of 2 - 48 tokens: 1.000 in the mean).
+// Q4 gate/up of 2 x 6144 x 2048, 33 tokens, is off by 1.52e-7, 1.63e-7 in chains of
+// a whole set, 1.65e-7 in slices of 16 blocks each one chain; the 12B gate/up of 16
+// tokens by 2.34e-7 with one chain per slice of 60.  It takes no measurable time.
 //
 // AF (the o and down inputs, and the kernel-level f32 entry points): A comes
 // as f32 rows, and the staging splits each token's slice itself, with a
@@ -1332,6 +1369,10 @@ __device__ __forceinline__ void stream_gemm(const _Float16* __restrict__ Ax,
           for (int e = 0; e < 4; e++) acc[h][e] += d[(p / 4) & 1][p % 4] * t[h][e];
           // (pinned here: put off, the FMAs keep every block's sums in registers)
           asm volatile("" : "+v"(acc[h]));
+          if (p == SB / 2 - 1) {
+            total[h] += acc[h];
+            acc[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+          }
         }
       }
     }

@@ -281,12 +281,12 @@ def test_prefill_stream_cuts(gpu, monkeypatch, mode, T, N, K, cut):
         assert_close(out[:T].view(np.float32), ref, rtol=rtol, what="streamed, cut %s" % cut)
 
 
-# The f32 sums over K: runs of 16 blocks added up by themselves.  Whole activations
+# The f32 sums over K: runs of 8 blocks added up by themselves.  Whole activations
 # (their lo halves are zero) and whole weights make every block's sum exact, so
 # what differs from the fp64 product is the rounding of the additions alone.  One
 # of them is off by 2^-23 / sqrt(12) of its binade, 2.5e-8 of its result in the
 # rms; a chain of n like terms by 2.5e-8 sqrt(n / 2) of its sum; runs, their sums
-# and the planes make n + ... of 16, blocks / 16 / planes and planes.  A quarter
+# and the planes make n + ... of 8, blocks / 8 / planes and planes.  A quarter
 # above that fails a chain over all of K (1.6e-7 to 2.0e-7 here).
 @pytest.mark.parametrize("mode", [gh.QUANT_Q4, gh.QUANT_Q8])
 @pytest.mark.parametrize("T,K,env,planes", [
@@ -301,7 +301,29 @@ def test_prefill_sums_in_runs(gpu, monkeypatch, mode, T, K, env, planes):
     gpu.prefill_gemm(mode, W, A, C, T, N, K)
     ref = a.astype(np.float64) @ deq.T
     err = np.linalg.norm(C.read(np.float32, T * N).reshape(T, N) - ref) / np.linalg.norm(ref)
-    n = 16 + K / 32 / 16 / planes + planes
+    n = 8 + K / 32 / 8 / planes + planes
+    assert err <= 1.25 * 2.53e-8 * np.sqrt(n / 2), (err, n)
+
+
+# The wide tile's in the same way, unsplit: runs of 16 blocks for more than 16
+# groups of four, of 8 for more than 4, else of 4; in the two largest tiles only
+# `share` of the rows, the others one chain over K.  (One chain in the other
+# tiles fails the bound: 1.9e-7 or more of 1.1e-7 at K = 3840.)
+@pytest.mark.parametrize("mode", [gh.QUANT_Q4, gh.QUANT_Q8])
+@pytest.mark.parametrize("K,run", [(3840, 16), (2048, 8), (512, 4)])
+@pytest.mark.parametrize("tile,T,share", [
+    ("1,1,128", 64, 1), ("2,1,128", 128, 1), ("3,1,128", 192, 1), ("1,1,256", 64, 1),
+    ("2,1,256", 120, 1), ("3,1,256", 192, 1 / 3), ("4,1,256", 256, 1 / 8)])
+def test_prefill_wide_sums_in_runs(gpu, monkeypatch, mode, K, run, tile, T, share):
+    monkeypatch.setenv("GH_PF_WIDE", tile)
+    N = 512
+    wq, deq = quantized(N, K, mode, 397)
+    a = np.random.default_rng(398).integers(-8, 9, (T, K)).astype(np.float32)
+    W, A, C = gpu.upload(wq), gpu.upload(a), gpu.alloc(T * N * 4)
+    gpu.prefill_gemm(mode, W, A, C, T, N, K)
+    ref = a.astype(np.float64) @ deq.T
+    err = np.linalg.norm(C.read(np.float32, T * N).reshape(T, N) - ref) / np.linalg.norm(ref)
+    n = share * (run + K / 32 / run) + (1 - share) * K / 32
     assert err <= 1.25 * 2.53e-8 * np.sqrt(n / 2), (err, n)
 
 
