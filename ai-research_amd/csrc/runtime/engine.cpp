@@ -400,9 +400,11 @@ uint32_t stream_kr_max(const gh_context* ctx, uint32_t T, uint32_t nw) {
 // 15360 rows by 1536 - 15360, 3 - 48 tokens) this takes one 1.1% behind the
 // best in the mean, 12% at worst.  Four waves serve narrow products: W_o of 16
 // tokens (3840 x 4096) 11.4 us on 120 workgroups of eight waves, 10.0 on 240 of
-// four.
-StreamCut stream_cut(const gh_context* ctx, gh_quant_mode mode, bool pair, uint32_t T, uint32_t N,
-                     uint32_t nb) {
+// four.  `sum`: planes are summed by a launch of their own (2.5-3 us, 32 of
+// these units), which slices of a small product do not repay: 256 x 512 of 16
+// tokens 10.4 us in two slices, 7.0 in one.
+StreamCut stream_cut(const gh_context* ctx, gh_quant_mode mode, bool pair, bool sum, uint32_t T,
+                     uint32_t N, uint32_t nb) {
   const uint32_t cus = (uint32_t)ctx->num_cus, units = (N + 15) / 16;
   StreamCut best;
   if (const char* env = getenv("GH_PF_STREAM")) {
@@ -425,7 +427,7 @@ StreamCut stream_cut(const gh_context* ctx, gh_quant_mode mode, bool pair, uint3
         const uint32_t wgs = ((units + nw * rgw - 1) / (nw * rgw)) * nz;
         const double rounds = (wgs + cus - 1) / cus;
         double cost = rounds * (6.45 + 0.02 * kr * T / nw + passes * nw * rgw * ((kr + sb - 1) / sb));
-        if (nz > 1) cost += 0.3 + 0.6 * nz * (pair ? 2 : 1) * T * (double)N * 8 / 4e6;
+        if (nz > 1) cost += (sum ? 32 : 0.3) + 0.6 * nz * (pair ? 2 : 1) * T * (double)N * 8 / 4e6;
         if (best.kr == 0 || cost < least) {
           least = cost;
           best = StreamCut{kr, rgw, nw};
@@ -436,15 +438,13 @@ StreamCut stream_cut(const gh_context* ctx, gh_quant_mode mode, bool pair, uint3
   return best;
 }
 
-gh_status launch_prefill_stream(gh_context* ctx, gh_quant_mode mode, const void* W0,
+gh_status launch_prefill_stream(gh_context* ctx, const StreamCut& cut, gh_quant_mode mode, const void* W0,
                                 const void* W1, const void* Ax, const float* rs, float* C,
                                 uint32_t T, uint32_t N, uint32_t K, const float** planes,
                                 uint32_t* nplanes, bool af) {
   const bool pair = W1 != nullptr;
   const uint32_t nmat = pair ? 2u : 1u;
   const uint32_t nb = K / 32, cus = (uint32_t)ctx->num_cus;
-  const StreamCut cut = stream_cut(ctx, mode, pair, T, N, nb);
-  if (cut.kr == 0) return fail(GH_ERR_UNSUPPORTED, "prefill GEMM: stream slice exceeds LDS");
   uint32_t KR = cut.kr, RGW = cut.rgw;
   const uint32_t nz = (nb + KR - 1) / KR, units = (N + 15) / 16;
   const std::string kname = std::string(pair ? "gh_pf_sgateup_" : "gh_pf_sgemm_") +
@@ -481,14 +481,14 @@ gh_status launch_prefill_stream(gh_context* ctx, gh_quant_mode mode, const void*
 // / 53.5; bf16 gate/up of 16 tokens 53-56 / 53, 32 tokens 69 / 58; Q4 down of
 // 48 tokens 33 / 36; bf16 down of 32 tokens 38 / 39, 40 tokens 44 / 40.
 bool stream_ok(const gh_context* ctx, gh_quant_mode mode, uint32_t T, uint32_t N, uint32_t K,
-               const void* W0, const void* W1) {
+               const void* W0, const void* W1, bool sum, StreamCut* cut) {
   const bool bf16 = mode == GH_QUANT_NONE;
   uint32_t tmax = W1 ? (bf16 ? 16u : mode == GH_QUANT_Q4 ? 40u : 48u) : (bf16 ? 32u : 48u);
   if (const char* env = getenv("GH_PF_STREAM_MAX")) tmax = std::min(tmax, (uint32_t)atoi(env));
   return T <= tmax && K % 128 == 0 &&
          !((reinterpret_cast<uintptr_t>(W0) | reinterpret_cast<uintptr_t>(W1 ? W1 : W0)) & 15) &&
-         stream_cut(ctx, mode, W1 != nullptr, T, N, K / 32).kr != 0 &&
-         getenv("GH_PF_NO_STREAM") == nullptr;
+         getenv("GH_PF_NO_STREAM") == nullptr &&
+         (*cut = stream_cut(ctx, mode, W1 != nullptr, sum, T, N, K / 32)).kr != 0;
 }
 
 // ---- the wide tile GEMM (gh_pf_wgemm_* / gh_pf_wgateup_*) ----
@@ -615,8 +615,9 @@ gh_status launch_prefill_gemm_split(gh_context* ctx, gh_quant_mode mode, const v
                                 "(16-byte for bf16 rows)");
   const bool pair = W1 != nullptr;
   if (pair && planes) return fail(GH_ERR_INVALID, "prefill GEMM: unsummed planes of a gate/up pair");
-  if (stream_ok(ctx, mode, T, N, K, W0, W1))
-    return launch_prefill_stream(ctx, mode, W0, W1, Ax, rs, C, T, N, K, planes, nplanes, false);
+  StreamCut cut;
+  if (stream_ok(ctx, mode, T, N, K, W0, W1, planes == nullptr, &cut))
+    return launch_prefill_stream(ctx, cut, mode, W0, W1, Ax, rs, C, T, N, K, planes, nplanes, false);
   // Longer batches take the wide tile, 1.02-1.75x the speed of the tiles below
   // wherever both were measured (wide_shape).  Those stay for K that is no
   // multiple of 128 and for weights that are not 16-byte aligned; their rules'
@@ -766,8 +767,9 @@ gh_status launch_prefill_gemm(gh_context* ctx, gh_quant_mode mode, const void* W
     return fail(GH_ERR_INVALID, "prefill GEMM: W null or misaligned (4 bytes; 16 for bf16 rows)");
   if (W1 && planes) return fail(GH_ERR_INVALID, "prefill GEMM: unsummed planes of a gate/up pair");
   // a short batch's streamed GEMM splits the f32 rows as it stages them
-  if (stream_ok(ctx, mode, T, N, K, W0, W1))
-    return launch_prefill_stream(ctx, mode, W0, W1, A, nullptr, C, T, N, K, planes, nplanes, true);
+  StreamCut cut;
+  if (stream_ok(ctx, mode, T, N, K, W0, W1, planes == nullptr, &cut))
+    return launch_prefill_stream(ctx, cut, mode, W0, W1, A, nullptr, C, T, N, K, planes, nplanes, true);
   const size_t ax_bytes = (size_t)T * K * 4;  // 2 K halves per row
   gh_status st = ctx->ensure_zeroed(&ctx->half_scratch, &ctx->half_scratch_bytes,
                                     ax_bytes + (size_t)T * sizeof(float));
