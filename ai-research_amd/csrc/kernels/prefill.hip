@@ -43,6 +43,7 @@
 #include <stdint.h>
 
 #include "../common/load_lds.h"
+#include "../common/wide_lds.h"
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -503,7 +504,7 @@ struct Unpack {
 // 8 g + 7, g = lane / 16); pair: two of the operand's eight halves.
 struct WQ4 {
   static constexpr bool kBf16 = false;
-  static constexpr int kChunks = 5, kRaw = 1;
+  static constexpr int kChunks = WIDE_CHUNKS_Q4, kRaw = 1;
   static constexpr int per(int rows, int j) { return j == 0 ? rows / 128 : j == 1; }
   __device__ static void raw(const uint8_t* row, uint32_t g, uint32_t* w, float* d) {
     const uint32_t* p = reinterpret_cast<const uint32_t*>(row);
@@ -529,7 +530,7 @@ struct WQ4 {
 };
 struct WQ8 {
   static constexpr bool kBf16 = false;
-  static constexpr int kChunks = 9, kRaw = 2;
+  static constexpr int kChunks = WIDE_CHUNKS_Q8, kRaw = 2;
   static constexpr int per(int rows, int j) { return j < 2 ? (rows == 256 ? 3 : 2) - j : 0; }
   __device__ static void raw(const uint8_t* row, uint32_t g, uint32_t* w, float* d) {
     const uint32_t* p = reinterpret_cast<const uint32_t*>(row);
@@ -547,7 +548,7 @@ struct WQ8 {
 };
 struct WBf16 {
   static constexpr bool kBf16 = true;
-  static constexpr int kChunks = 4, kRaw = 4;
+  static constexpr int kChunks = WIDE_CHUNKS_BF16, kRaw = 4;
   static constexpr int per(int rows, int) { return rows / 128; }
   __device__ static void raw(const uint8_t* chunk, uint32_t, uint32_t* w, float*) {
     const u32x4 v = *reinterpret_cast<const u32x4*>(chunk);
@@ -557,31 +558,16 @@ struct WBf16 {
   __device__ static uint32_t pair(const uint32_t* w, int p, const Unpack&) { return w[p]; }
 };
 
-// LDS: kStages steps of A, kGroups groups of four blocks of W (bf16: a step's W
-// beside its A), and a place for the unused part of a group's last load.
-template <class F, int TM, int BR>
-struct WideLds {
-  static constexpr uint32_t kMax = 160 * 1024;
-  static constexpr uint32_t kA = 64 * TM * 128;
-  static constexpr uint32_t kB = BR * 16 * F::kChunks;
-  static constexpr uint32_t kPad = F::kBf16 ? 0 : 1024;
-  static constexpr int kGroups = F::kBf16 ? 0 : 3 * kA + 3 * kB + kPad <= kMax ? 3 : 2;
-  static constexpr int kFit = (kMax - kPad - kGroups * kB) / (kA + (F::kBf16 ? kB : 0));
-  static constexpr int kStages = kFit < 5 ? kFit : 5;
-  static constexpr int kBStages = F::kBf16 ? kStages : kGroups;
-  static constexpr uint32_t kBytes = kStages * kA + kBStages * kB + kPad;
-};
-
 template <class F, int TM, int NMAT, int BR>
 __device__ __forceinline__ void wide_tile(const _Float16* __restrict__ Ax,
                                           const float* __restrict__ rs,
                                           const uint8_t* __restrict__ W0,
                                           const uint8_t* __restrict__ W1, float* __restrict__ C,
                                           uint32_t T, uint32_t N, uint32_t K) {
-  using L = WideLds<F, TM, BR>;
+  constexpr WideLds L = wide_lds(F::kBf16, F::kChunks, TM, BR);
   constexpr int NA = TM;  // A pieces per thread and step (64 TM rows x 8 / 512)
-  constexpr int NS = L::kStages;
-  constexpr int NG = L::kGroups;
+  constexpr int NS = L.stages;
+  constexpr int NG = L.groups;
   constexpr uint32_t BN = BR / NMAT;          // columns of C
   constexpr int WN = 4;                       // wavefronts in N (2 in M)
   constexpr int MT = 2 * TM, NT = BR / 64;    // 16 x 16 blocks of a wavefront
@@ -615,7 +601,7 @@ __device__ __forceinline__ void wide_tile(const _Float16* __restrict__ Ax,
     const uint8_t* base = a_base + (size_t)min(step, s_end - 1) * 128;
 #pragma unroll
     for (int i = 0; i < NA; i++)
-      load_lds16(a_off[i], base, lds0 + st * L::kA + 8192 * i + 1024 * wave);
+      load_lds16(a_off[i], base, lds0 + st * L.a + 8192 * i + 1024 * wave);
   };
   // W: piece c of four blocks is row c / kChunks, part c % kChunks (bf16: of a
   // step, row c / 4, position c % 4 from chunk (c % 4) ^ swizzle)
@@ -630,14 +616,14 @@ __device__ __forceinline__ void wide_tile(const _Float16* __restrict__ Ax,
     b_src[i] = W + (size_t)min(n0 + r % BN, N - 1) * row_bytes +
                16 * (F::kBf16 ? part ^ bswz(r) : part);
   }
-  constexpr uint32_t kB0 = NS * L::kA, kPad0 = kB0 + L::kBStages * L::kB;
+  constexpr uint32_t kB0 = NS * L.a, kPad0 = kB0 + (F::kBf16 ? NS : NG) * L.b;
   auto load_b = [&](int i, uint32_t unit, uint32_t st) {  // unit: a group of four (bf16: a step)
     const uint32_t step_bytes = F::kBf16 ? 64 : 16 * F::kChunks;
     const uint32_t last = (F::kBf16 ? s_end : q_end) - 1;
     // a group's last load may need fewer wavefronts: the others' goes to the pad
     const bool pad = 512u * i + 64u * wave >= (uint32_t)BR * F::kChunks;
     load_lds16(b_src[i] + (size_t)min(unit, last) * step_bytes,
-               lds0 + (pad ? kPad0 : kB0 + st * L::kB + 8192 * i + 1024 * wave));
+               lds0 + (pad ? kPad0 : kB0 + st * L.b + 8192 * i + 1024 * wave));
   };
 
   const uint32_t wm = (wave / WN) * (16 * MT), wn = wave % WN, g = lane >> 4, l16 = lane & 15;
@@ -654,14 +640,14 @@ __device__ __forceinline__ void wide_tile(const _Float16* __restrict__ Ax,
 #pragma unroll
     for (int c = 0; c < NT; c++) {
       if constexpr (F::kBf16)
-        F::raw(pf_wide + kB0 + bst * L::kB + b_row(c) * 64 + 16 * (g ^ bswz(l16)), g, r[c], &d[c]);
+        F::raw(pf_wide + kB0 + bst * L.b + b_row(c) * 64 + 16 * (g ^ bswz(l16)), g, r[c], &d[c]);
       else
-        F::raw(pf_wide + kB0 + bst * L::kB + b_row(c) * (16 * F::kChunks) + j * (4 * F::kChunks), g, r[c], &d[c]);
+        F::raw(pf_wide + kB0 + bst * L.b + b_row(c) * (16 * F::kChunks) + j * (4 * F::kChunks), g, r[c], &d[c]);
     }
   };
   auto read_a = [&](half8 (&a)[2], uint32_t st, int i) {
-    a[0] = *reinterpret_cast<const half8*>(pf_wide + st * L::kA + a_hi + 2048 * i);
-    a[1] = *reinterpret_cast<const half8*>(pf_wide + st * L::kA + a_lo + 2048 * i);
+    a[0] = *reinterpret_cast<const half8*>(pf_wide + st * L.a + a_hi + 2048 * i);
+    a[1] = *reinterpret_cast<const half8*>(pf_wide + st * L.a + a_lo + 2048 * i);
   };
 
   f32x4 acc[MT][NT];
@@ -860,8 +846,8 @@ __device__ __forceinline__ void wide_tile(const _Float16* __restrict__ Ax,
   }
 }
 
-// (two wavefronts per SIMD at least; the small tiles' registers and LDS let a
-// second workgroup onto a CU)
+// (two wavefronts per SIMD at least; the registers and LDS of the 64 x 128 tile,
+// but for Q8 weights, let a second workgroup onto a CU)
 #define GH_WIDE_TM(FMT, F, TM, BR)                                                            \
   extern "C" __global__ __launch_bounds__(PF_WIDE_NT) __attribute__((amdgpu_waves_per_eu(2)))  \
   void gh_pf_wgemm_##FMT##_m##TM##_n##BR##_k(const _Float16* Ax, const float* rs,              \

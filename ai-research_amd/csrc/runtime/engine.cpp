@@ -9,6 +9,7 @@
 
 #include "runtime.hpp"
 #include "../common/stream_args.h"
+#include "../common/wide_lds.h"
 
 using gh::fail;
 
@@ -498,24 +499,23 @@ struct WideShape {
   uint32_t tm = 0, br = 256, nz = 1;
 };
 
-// LDS bytes of a tile (WideLds in prefill.hip)
-unsigned wide_lds(gh_quant_mode mode, uint32_t tm, uint32_t br) {
-  const unsigned max = 160 * 1024, a = 64 * tm * 128;
-  const unsigned b = br * 16 * (mode == GH_QUANT_Q4 ? 5 : mode == GH_QUANT_Q8 ? 9 : 4);
-  if (mode == GH_QUANT_NONE) return std::min(5u, max / (a + b)) * (a + b);
-  const unsigned pad = 1024, groups = 3 * a + 3 * b + pad <= max ? 3 : 2;
-  return std::min(5u, (max - pad - groups * b) / a) * a + groups * b + pad;
+WideLds wide_lds_of(gh_quant_mode mode, uint32_t tm, uint32_t br) {
+  const uint32_t chunks = mode == GH_QUANT_Q4 ? WIDE_CHUNKS_Q4 : mode == GH_QUANT_Q8 ? WIDE_CHUNKS_Q8 : WIDE_CHUNKS_BF16;
+  return wide_lds(mode == GH_QUANT_NONE, chunks, tm, br);
 }
 
-// The cheapest tile and split by a cost in us: rounds of workgroups over the
-// CUs (the 64 x 128 tile fits a CU twice) times steps of one block, plus the
-// split planes' traffic.  The constants are fitted to 297 measured products
-// (three weight modes, 9 shapes of 2048 - 15360 rows by 1536 - 15360, 11
-// lengths of 49 - 512 tokens, up to 30 tiles and splits each): the tile taken
-// is 1.0% behind the best one in the mean and 14% at worst, and ahead of the
-// 64- and 128-row tiles of one K block per barrier in every one of them
-// (1.02 to 1.75x).  GH_PF_WIDE="tm,nz,br" forces one.
-WideShape wide_shape(const gh_context* ctx, bool pair, uint32_t T, uint32_t N, uint32_t K) {
+// The cheapest tile and split by a cost that ranks them (in units near a us, but
+// no estimate of the time): rounds of workgroups over the CUs (the 64 x 128 tile
+// fits a CU twice, but for Q8 weights) times steps of one block, plus the split
+// planes' traffic.  The constants are fitted to measured products (three weight
+// modes, 9 shapes of 2048 - 15360 rows by 1536 - 15360, 11 lengths of 49 - 512
+// tokens, up to 30 tiles and splits each): over 297 of them the tile taken is 1.3%
+// behind the best one in the mean and 19% at worst.  The 64- and 128-row tiles of
+// one K block per barrier take 1.21 times as long in the mean; they were ahead in 3
+// of 165 products (by 1 - 5%, 2944 x 9600 of 400 and 512 tokens).
+// GH_PF_WIDE="tm,nz,br" forces one.
+WideShape wide_shape(const gh_context* ctx, gh_quant_mode mode, bool pair, uint32_t T, uint32_t N,
+                     uint32_t K) {
   const uint32_t cus = (uint32_t)ctx->num_cus, nq = K / 128;
   WideShape best;
   if (const char* env = getenv("GH_PF_WIDE")) {
@@ -530,7 +530,7 @@ WideShape wide_shape(const gh_context* ctx, bool pair, uint32_t T, uint32_t N, u
     for (uint32_t tm = 1; tm <= (br == 128 ? 3u : 4u); tm++) {
       const uint32_t bn = pair ? br / 2 : br, rows = 64 * tm;
       const uint64_t tiles = (uint64_t)((N + bn - 1) / bn) * ((T + rows - 1) / rows);
-      const bool twice = br == 128 && tm == 1;
+      const bool twice = br == 128 && tm == 1 && 2 * wide_lds_of(mode, tm, br).bytes <= WIDE_LDS_MAX;
       const uint32_t zmax = (uint32_t)std::min<uint64_t>(std::min(nq, 64u), 2 * cus / tiles);
       for (uint32_t nz = 1; nz <= std::max(1u, zmax); nz++) {
         const double load = (double)(tiles * nz) / cus;
@@ -560,7 +560,7 @@ gh_status launch_prefill_wide(gh_context* ctx, gh_quant_mode mode, const void* W
                               const void* Ax, const float* rs, float* C, uint32_t T, uint32_t N,
                               uint32_t K, const float** planes, uint32_t* nplanes) {
   const bool pair = W1 != nullptr;
-  const WideShape sh = wide_shape(ctx, pair, T, N, K);
+  const WideShape sh = wide_shape(ctx, mode, pair, T, N, K);
   const uint32_t bn = pair ? sh.br / 2 : sh.br, nmat = pair ? 2u : 1u;
   uint32_t nz = sh.nz;
   float* out = C;
@@ -574,7 +574,7 @@ gh_status launch_prefill_wide(gh_context* ctx, gh_quant_mode mode, const void* W
                            (mode == GH_QUANT_Q8 ? "q8" : mode == GH_QUANT_NONE ? "bf16" : "q4") +
                            "_m" + std::to_string(sh.tm) + "_n" + std::to_string(sh.br) + "_k";
   const dim3 grid((N + bn - 1) / bn, (T + 64 * sh.tm - 1) / (64 * sh.tm), nz);
-  const unsigned lds = wide_lds(mode, sh.tm, sh.br);
+  const unsigned lds = wide_lds_of(mode, sh.tm, sh.br).bytes;
   gh_status st;
   if (pair) {
     void* args[] = {const_cast<void**>(&Ax), const_cast<float**>(&rs), const_cast<void**>(&W0),
@@ -618,7 +618,7 @@ gh_status launch_prefill_gemm_split(gh_context* ctx, gh_quant_mode mode, const v
   StreamCut cut;
   if (stream_ok(ctx, mode, T, N, K, W0, W1, planes == nullptr, &cut))
     return launch_prefill_stream(ctx, cut, mode, W0, W1, Ax, rs, C, T, N, K, planes, nplanes, false);
-  // Longer batches take the wide tile, 1.02-1.75x the speed of the tiles below
+  // Longer batches take the wide tile, which is faster than the tiles below nearly
   // wherever both were measured (wide_shape).  Those stay for K that is no
   // multiple of 128 and for weights that are not 16-byte aligned; their rules'
   // figures are of the 12B products, which they served before the wide tile.

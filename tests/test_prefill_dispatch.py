@@ -33,3 +33,14 @@ def test_small_products_are_one_launch(checks, mode, pair, N, K):
     most = {"q4": (48, 40), "q8": (48, 48), "bf16": (32, 16)}[mode][pair]
     for T, calls in zip((2, 8, 16, most), launches(checks, [(mode, pair, T, N, K) for T in (2, 8, 16, most)])):
         assert len(calls) == 1 and calls[0][1][2] == 1, (T, calls)
+
+
+# The 64 x 128 tile fits a CU twice with Q4 and bf16 weights, not with Q8 ones: 352
+# workgroups of an unsplit gate/up are one and a half rounds or two.  A grid's LDS
+# is that of the layout the kernel is compiled with (csrc/common/wide_lds.h).
+@pytest.mark.parametrize("mode,lds", [("q4", 5 * 8192 + 3 * 10240 + 1024), ("q8", 5 * 8192 + 3 * 18432 + 1024),
+                                      ("bf16", 5 * (8192 + 8192))])
+def test_wide_tile_residency(checks, mode, lds):
+    wide = [c for c in launches(checks, [(mode, 1, 64, 11264, 6144)])[0] if "wgateup" in c[0]]
+    assert [c[0] for c in wide] == ["gh_pf_wgateup_%s_m1_n128_k" % mode] and wide[0][3] == lds
+    assert (2 * lds <= 160 * 1024) == (mode != "q8")
