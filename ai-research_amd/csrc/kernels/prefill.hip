@@ -467,19 +467,21 @@ GH_GEMM_PAIR_W8(gh_pf_gateup_q4_m128_n64, Q4W, 128, 64, 1, true, _s_w8)
 // Sums: an fp32 chain over all of an unsplit K is off by more than the split
 // tiles' shorter ones, so runs of blocks (16 for long K) are chains of their own
 // whose sums are added up in second registers.  The tiles of 192 and 256 tokens
-// by 256 rows have registers for only 2 of 6 and 1 of 8 of their 16-row blocks
+// by 256 rows have registers for only 3 of 6 and 1 of 8 of their 16-row blocks
 // (bf16: for none, but its 16-bit activations are 10 times further off); they
 // take the products that were unsplit before.  Against 64 bits, tile GEMM / one
 // chain / runs, Q4: gate/up 2 x 15360 x 3840 of 64, 128 and 333 tokens 2.05 / 3.09
-// / 1.72e-7, 2.35 / 3.10 / 1.72e-7 and 2.95 / 3.11 / 2.66e-7, down 3840 x 15360 of
-// 128 tokens 1.43 / 1.65 / 1.17e-7.  It takes 2.4% in the mean of 165 products.
+// / 1.74e-7, 2.35 / 3.10 / 1.73e-7 and 2.95 / 3.11 / 2.42e-7, down 3840 x 15360 of
+// 128 tokens 1.43 / 1.65 / 1.18e-7.  It takes 1.1% in the mean of 165 products: a
+// run is a loop of its own, as a branch or selects in one loop over K cost the
+// larger tiles registers or 5%.
 //
 // Measured, 12B gate/up of 512 tokens, tile GEMM -> this (the whole call, its
-// activation split included): Q4 275 -> 206 us (1170 TFLOP/s executed), Q8 295 ->
-// 217, bf16 272 -> 187.  Within a whole prompt's trace the Q4 kernel takes 224 us,
+// activation split included): Q4 281 -> 209 us (1160 TFLOP/s executed), Q8 297 ->
+// 219, bf16 269 -> 189.  Within a whole prompt's trace the Q4 kernel takes 224 us,
 // at a lower clock.  Timing-only copies took 11% less without the loads, 22%
 // without the LDS reads of A as well.  The gate/up of 128 tokens (TM 2, BR 128,
-// which keeps K unsplit) 89 -> 74 us, of 64 tokens 62 -> 53 us.
+// which keeps K unsplit) 89 -> 73 us, of 64 tokens 61 -> 52 us.
 // ---------------------------------------------------------------------------
 #define PF_WIDE_NT 512
 
@@ -656,7 +658,7 @@ __device__ __forceinline__ void wide_tile(const _Float16* __restrict__ Ax,
 #pragma unroll
     for (int c = 0; c < NT; c++) acc[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
   // the runs' sums: of as many of the 16-row blocks as registers are left for
-  constexpr int MR = TM <= 2 || BR == 128 ? MT : F::kBf16 ? 0 : TM == 3 ? 2 : 1;
+  constexpr int MR = TM <= 2 || BR == 128 ? MT : F::kBf16 ? 0 : TM == 3 ? 3 : 1;
   f32x4 runs[MR > 0 ? MR : 1][NT];
 #pragma unroll
   for (int i = 0; i < MR; i++)
@@ -706,102 +708,100 @@ __device__ __forceinline__ void wide_tile(const _Float16* __restrict__ Ax,
 #pragma unroll
     for (int p = 0; p < 4; p++) b[c][p] = F::pair(raw[c], p, uc);
 
-  for (uint32_t q = q_begin; q < q_end; q++) {
-    int nload = 0;
+  for (uint32_t q = q_begin; q < q_end;) {
+    const uint32_t q_run = MR > 0 ? min(q + run, q_end) : q_end;
+    for (; q < q_run; q++) {
+      int nload = 0;
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-      // loads of a later step's operands, into the stage that the previous
-      // step read (every wave has passed a barrier since)
-      uint32_t nst = st + NS - 1;
-      nst = nst >= (uint32_t)NS ? nst - NS : nst;
-      if constexpr (F::kBf16) {
-#pragma unroll
-        for (int i = 0; i < NB; i++) load_b(i, step + NS - 1, nst);
-      } else {
-        const uint32_t nbq = bq == 0 ? NG - 1 : bq - 1;
-#pragma unroll
-        for (int p = 0; p < F::per(BR, j); p++) load_b(nload + p, q + NG - 1, nbq);
-        nload += F::per(BR, j);
-      }
-      load_a(step + NS - 1, nst);
-      const uint32_t sn = st + 1 == (uint32_t)NS ? 0 : st + 1;
-      // quantized: the next step's words are in LDS already (of the next group
-      // since the barrier of this group's third step); they are unpacked
-      // between the MFMAs
-      if constexpr (!F::kBf16) read_raw(raw, dn, j < 3 ? bq : bq + 1 == (uint32_t)NG ? 0 : bq + 1, (j + 1) & 3);
-#pragma unroll
-      for (int i = 0; i < MT; i++) {
-        if (i == MT - 1) {
-          // The next step's operands have landed for every wave: of the loads
-          // issued since, those of the last NS - 2 steps may be in flight; with
-          // two groups of W, in a group's third step only the A of two steps
-          // (the next group's last W went out in the second, ahead of that A).
-          constexpr int flight = (NS - 2) * per_step;
-          if (!F::kBf16 && NG == 2 && j == 2)
-            wait_loads_barrier<flight < 2 * NA ? flight : 2 * NA>();
-          else
-            wait_loads_barrier<flight>();
-          if constexpr (F::kBf16) read_raw(raw, dn, sn, 0);
-          read_a(a[(i + 1) & 1], sn, 0);
-        } else {
-          read_a(a[(i + 1) & 1], st, i + 1);
-        }
-        // (the compiler would sink the reads to just ahead of their use)
-        __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-        for (int h = 0; h < 2; h++)
-#pragma unroll
-          for (int c = 0; c < NT; c++) {
-            if constexpr (F::kBf16) {
-              acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-                  __builtin_bit_cast(bf16x8, a[i & 1][h]), __builtin_bit_cast(bf16x8, b[c]), acc[i][c], 0, 0, 0);
-            } else {
-              // one MFMA, then two scale FMAs of the previous 16 rows and a
-              // share of the unpacking: an MFMA that finds the matrix pipe
-              // busy holds up the SIMD's vector instructions too
-              t[i & 1][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                  a[i & 1][h], __builtin_bit_cast(half8, b[c]), h ? t[i & 1][c] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-              const int slot = h * NT + c;
-#pragma unroll
-              for (int e = 2 * slot; e < 2 * slot + 2; e++)
-                acc[(i + MT - 1) % MT][e / 4][e % 4] += (i ? d : dp)[e / 4] * t[(i + 1) & 1][e / 4][e % 4];
-              if (i > 0) {
-                constexpr int slots = (MT - 1) * 2 * NT, pairs = 4 * NT;
-                const int u = (i - 1) * 2 * NT + slot;
-#pragma unroll
-                for (int p = u * pairs / slots; p < (u + 1) * pairs / slots; p++)
-                  bn[p / 4][p % 4] = F::pair(raw[p / 4], p % 4, uc);
-              }
-            }
-          }
-      }
-#pragma unroll
-      for (int c = 0; c < NT; c++) {
+      for (int j = 0; j < 4; j++) {
+        // loads of a later step's operands, into the stage that the previous
+        // step read (every wave has passed a barrier since)
+        uint32_t nst = st + NS - 1;
+        nst = nst >= (uint32_t)NS ? nst - NS : nst;
         if constexpr (F::kBf16) {
 #pragma unroll
-          for (int p = 0; p < 4; p++) b[c][p] = raw[c][p];
+          for (int i = 0; i < NB; i++) load_b(i, step + NS - 1, nst);
         } else {
-          b[c] = bn[c];
-          dp[c] = d[c];
-          d[c] = dn[c];
+          const uint32_t nbq = bq == 0 ? NG - 1 : bq - 1;
+#pragma unroll
+          for (int p = 0; p < F::per(BR, j); p++) load_b(nload + p, q + NG - 1, nbq);
+          nload += F::per(BR, j);
         }
-      }
-      step++;
-      st = sn;
-    }
-    bq = bq + 1 == (uint32_t)NG ? 0 : bq + 1;
-    const bool end = ((q + 1 - q_begin) & (run - 1)) == 0;
-    if (MR < MT || end) {  // (the larger tiles: selects, a branch would spill)
+        load_a(step + NS - 1, nst);
+        const uint32_t sn = st + 1 == (uint32_t)NS ? 0 : st + 1;
+        // quantized: the next step's words are in LDS already (of the next group
+        // since the barrier of this group's third step); they are unpacked
+        // between the MFMAs
+        if constexpr (!F::kBf16) read_raw(raw, dn, j < 3 ? bq : bq + 1 == (uint32_t)NG ? 0 : bq + 1, (j + 1) & 3);
 #pragma unroll
-      for (int i = 0; i < MR; i++)
-#pragma unroll
-        for (int c = 0; c < NT; c++)
-#pragma unroll
-          for (int e = 0; e < 4; e++) {
-            runs[i][c][e] += end ? acc[i][c][e] : 0.f;
-            acc[i][c][e] = end ? 0.f : acc[i][c][e];
+        for (int i = 0; i < MT; i++) {
+          if (i == MT - 1) {
+            // The next step's operands have landed for every wave: of the loads
+            // issued since, those of the last NS - 2 steps may be in flight; with
+            // two groups of W, in a group's third step only the A of two steps
+            // (the next group's last W went out in the second, ahead of that A).
+            constexpr int flight = (NS - 2) * per_step;
+            if (!F::kBf16 && NG == 2 && j == 2)
+              wait_loads_barrier<flight < 2 * NA ? flight : 2 * NA>();
+            else
+              wait_loads_barrier<flight>();
+            if constexpr (F::kBf16) read_raw(raw, dn, sn, 0);
+            read_a(a[(i + 1) & 1], sn, 0);
+          } else {
+            read_a(a[(i + 1) & 1], st, i + 1);
           }
+          // (the compiler would sink the reads to just ahead of their use)
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int c = 0; c < NT; c++) {
+              if constexpr (F::kBf16) {
+                acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    __builtin_bit_cast(bf16x8, a[i & 1][h]), __builtin_bit_cast(bf16x8, b[c]), acc[i][c], 0, 0, 0);
+              } else {
+                // one MFMA, then two scale FMAs of the previous 16 rows and a
+                // share of the unpacking: an MFMA that finds the matrix pipe
+                // busy holds up the SIMD's vector instructions too
+                t[i & 1][c] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                    a[i & 1][h], __builtin_bit_cast(half8, b[c]), h ? t[i & 1][c] : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                const int slot = h * NT + c;
+#pragma unroll
+                for (int e = 2 * slot; e < 2 * slot + 2; e++)
+                  acc[(i + MT - 1) % MT][e / 4][e % 4] += (i ? d : dp)[e / 4] * t[(i + 1) & 1][e / 4][e % 4];
+                if (i > 0) {
+                  constexpr int slots = (MT - 1) * 2 * NT, pairs = 4 * NT;
+                  const int u = (i - 1) * 2 * NT + slot;
+#pragma unroll
+                  for (int p = u * pairs / slots; p < (u + 1) * pairs / slots; p++)
+                    bn[p / 4][p % 4] = F::pair(raw[p / 4], p % 4, uc);
+                }
+              }
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < NT; c++) {
+          if constexpr (F::kBf16) {
+#pragma unroll
+            for (int p = 0; p < 4; p++) b[c][p] = raw[c][p];
+          } else {
+            b[c] = bn[c];
+            dp[c] = d[c];
+            d[c] = dn[c];
+          }
+        }
+        step++;
+        st = sn;
+      }
+      bq = bq + 1 == (uint32_t)NG ? 0 : bq + 1;
     }
+#pragma unroll
+    for (int i = 0; i < MR; i++)
+#pragma unroll
+      for (int c = 0; c < NT; c++) {
+        runs[i][c] += acc[i][c];
+        acc[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
   }
   if constexpr (!F::kBf16) {
 #pragma unroll

@@ -313,7 +313,7 @@ def test_prefill_sums_in_runs(gpu, monkeypatch, mode, T, K, env, planes):
 @pytest.mark.parametrize("K,run", [(3840, 16), (2048, 8), (512, 4)])
 @pytest.mark.parametrize("tile,T,share", [
     ("1,1,128", 64, 1), ("2,1,128", 128, 1), ("3,1,128", 192, 1), ("1,1,256", 64, 1),
-    ("2,1,256", 120, 1), ("3,1,256", 192, 1 / 3), ("4,1,256", 256, 1 / 8)])
+    ("2,1,256", 120, 1), ("3,1,256", 192, 1 / 2), ("4,1,256", 256, 1 / 8)])
 def test_prefill_wide_sums_in_runs(gpu, monkeypatch, mode, K, run, tile, T, share):
     monkeypatch.setenv("GH_PF_WIDE", tile)
     N = 512
