@@ -27,11 +27,8 @@ def quantized(rows, cols, mode, seed):
     return wq, deq
 
 
-# (T, N, K): single row, ragged T and N, the 12B K, T past one 128-row tile,
-# and a long prompt's narrow product (128x128 tiles with K split 3 ways)
-# (512, 8192, 256): 256 tiles of 128x128, so the 128x64 tile runs (two per CU);
-# (96, 8192, 1024): one 128-row tile of 96 tokens, 64 tiles split 4 ways;
-# (300, 128, 1024): 256 tokens on the tiles, the last 44 streamed
+# (T, N, K): single row, ragged T and N, the 12B K, and long prompts' products of
+# few and many rows, streamed up to 48 (bf16: 32) tokens and on the wide tile above
 GEMM_SHAPES = [(1, 64, 128), (7, 96, 256), (64, 384, 3840), (130, 256, 512), (300, 128, 1024),
                (512, 3840, 1024), (512, 8192, 256), (96, 8192, 1024)]
 
@@ -47,10 +44,7 @@ def test_prefill_gemm(gpu, mode, T, N, K):
     assert_close(got, np.asarray(a, np.float64) @ deq.T, what="prefill GEMM")
 
 
-# (100, 8192, 1024): Q4 takes the 128x64 pair tile with K split (64 tiles of one
-# 128-row tile, half the CU count or more); (288, 512, 1024) and (300, 192, 3840):
-# the first 256 tokens on the tiles, the rest on the weight-streaming GEMM;
-# (352, 192, 1024): the rest of 96 tokens on the tiles
+# (streamed up to 40, Q8 48 and bf16 16 tokens, on the wide tile above)
 @pytest.mark.parametrize("mode", [gh.QUANT_Q4, gh.QUANT_Q8, gh.QUANT_NONE])
 @pytest.mark.parametrize("T,N,K", [(1, 64, 128), (45, 192, 512), (256, 512, 3840),
                                    (100, 8192, 1024), (288, 512, 1024), (300, 192, 3840),
@@ -67,14 +61,11 @@ def test_prefill_gate_up_geglu(gpu, mode, T, N, K):
     assert_close(got, ref, what="prefill GeGLU")
 
 
-# The 128x64 gate/up tile (gh_pf_gateup_q{4,8}_m128_n64_k1) runs when
-# ceil(N / 64) * ceil(T / 128) reaches the CU count (256): the 12B gate/up of
-# a 512-token prompt (960 tiles) and a ragged 129-token batch of exactly 256
-# tiles (its second 128-row tile holds one token).
+# The gate/up of many workgroups: the 12B one of a 512-token prompt, and a ragged
+# batch whose second 128 rows hold one token.
 @pytest.mark.parametrize("mode", [gh.QUANT_Q4, gh.QUANT_Q8, gh.QUANT_NONE])
 @pytest.mark.parametrize("T,N,K", [(512, 15360, 3840), (129, 8192, 512)])
 def test_prefill_gate_up_large_tiles(gpu, mode, T, N, K):
-    assert -(-N // 64) * -(-T // 128) >= 256
     gq, gdeq = quantized(N, K, mode, 340)
     uq, udeq = quantized(N, K, mode, 341)
     a = gh.synth_normal(T * K, 1, 342, 0.0, 1.0).reshape(T, K)
@@ -84,7 +75,7 @@ def test_prefill_gate_up_large_tiles(gpu, mode, T, N, K):
     a64 = np.asarray(a, np.float64)
     ref = nr.gelu64(a64 @ gdeq.T) * (a64 @ udeq.T)
     del gdeq, udeq
-    assert_close(got, ref, what="prefill GeGLU, 128x64 tiles")
+    assert_close(got, ref, what="prefill GeGLU, many tiles")
     for t in (0, T - 1):  # first and last rows, one of them alone in its tile
         assert_close(got[t], ref[t], what="prefill GeGLU row %d" % t)
 
@@ -139,6 +130,40 @@ def test_prefill_wide_tiles(gpu, monkeypatch, mode, T, N, K, force):
         result("tile GEMM, 4-byte aligned weights", a64 @ gdeq.T)
 
 
+# The tile GEMM's forms, which serve K off 128 (and weights off 16 bytes):
+# (pair, T, N, K, the kernel of Q4 rows, of the other two).  64 x 64 tiles, split
+# and not, 128 x 128 split, not split and 128 x 64, the pair's 128 x 64 in 8- and
+# 4-wave workgroups and (Q4) split, a rest past 256 tokens; N ragged in each.
+# tests/test_prefill_dispatch.py holds them to their kernels.
+TILE_SHAPES = [
+    (0, 49, 16350, 288, "gemm_m64_n64_k1", None), (0, 50, 200, 544, "gemm_m64_n64_k1_s", None),
+    (0, 96, 1000, 1056, "gemm_m128_n128_k1_s_w8", None), (0, 511, 16300, 160, "gemm_m128_n128_k1_w8", None),
+    (0, 512, 8150, 160, "gemm_m128_n64_k1_w8", None), (0, 300, 630, 288, "gemm_m128_n128_k1_w8", None),
+    (1, 100, 8150, 544, "gateup_m128_n64_k1_s_w8", "gateup_m64_n64_k1"), (1, 49, 200, 544, "gateup_m64_n64_k1_s", None),
+    (1, 129, 8150, 160, "gateup_m128_n64_k1_w8", None), (1, 509, 12390, 160, "gateup_m128_n64_k1", None)]
+
+
+@pytest.mark.parametrize("mode", [gh.QUANT_Q4, gh.QUANT_Q8, gh.QUANT_NONE])
+@pytest.mark.parametrize("shape", TILE_SHAPES, ids=lambda s: "-".join(map(str, s[:4])))
+def test_prefill_tile_forms(gpu, mode, shape):
+    # bound as in test_prefill_wide_tiles
+    pair, T, N, K = shape[:4]
+    gq, gdeq = quantized(N, K, mode, 410)
+    a = gh.synth_normal(T * K, 1, 412, 0.0, 1.0).reshape(T, K)
+    ref = np.asarray(a, np.float64) @ gdeq.T
+    W, A, C = gpu.upload(gq), gpu.upload(a), gpu.alloc((T + 64) * N * 4)
+    gpu.fill_u32(C, 0x7FC12345, (T + 64) * N)
+    if pair:
+        uq, udeq = quantized(N, K, mode, 411)
+        gpu.prefill_gate_up_geglu(mode, W, gpu.upload(uq), A, C, T, N, K)
+        ref = nr.gelu64(ref) * (np.asarray(a, np.float64) @ udeq.T)
+    else:
+        gpu.prefill_gemm(mode, W, A, C, T, N, K)
+    out = C.read(np.uint32, (T + 64) * N).reshape(T + 64, N)
+    assert np.all(out[T:] == 0x7FC12345)
+    assert_close(out[:T].view(np.float32), ref, rtol=1e-3 if mode == gh.QUANT_NONE else 2e-5, what="tile form")
+
+
 def test_prefill_gemm_row_range(gpu):
     # rows far outside fp16 range (1e6, 1e-7), a zero row and mixed magnitudes
     # within a row: the per-row power-of-two scale keeps every row exact to
@@ -188,13 +213,12 @@ def test_prefill_gemm_weight_scale_range(gpu):
         assert_close(got[:, n], ref[:, n], what="prefill GEMM weight row %d" % n)
 
 
-# Batches of at most 48 tokens with K a multiple of 128 run the
-# weight-streaming GEMM (16-token groups on the 16x16x32 MFMA; 8-wave
-# workgroups with two groups per wave from 17 tokens and three from 33, where
-# their LDS fits; K in slices staged in LDS, the slices' planes added in
-# order).  One token; 16; 17 and 32; 33, 40, 45 and 48 (narrower slices); a
-# ragged N; the 12B K values (3840, 4096, 15360); K of four quant blocks (one
-# slice, a partial weight set).  K = 160 and 49 tokens take the tile GEMM.
+# Batches of at most 48 tokens (a Q4 gate/up pair 40, bf16 32 and 16) with K a
+# multiple of 128 run the weight-streaming GEMM (16-token groups on the 16x16x32
+# MFMA; K in slices staged in LDS, the slices' planes added in order).  One token;
+# 16; 17 and 32; 33, 40, 45 and 48; a ragged N; the 12B K values (3840, 4096,
+# 15360); K of four quant blocks (one slice, a partial register set).  K = 160 takes
+# the tile GEMM, 49 tokens the wide tile.
 STREAM_SHAPES = [(1, 64, 128), (4, 100, 3840), (16, 256, 4096), (13, 96, 15360), (16, 48, 2048),
                  (9, 512, 128), (17, 96, 3840), (32, 200, 4096), (27, 64, 15360), (6, 40, 160),
                  (33, 64, 256), (40, 96, 3840), (48, 200, 4096), (45, 64, 15360), (49, 64, 256)]
@@ -251,15 +275,20 @@ def test_prefill_stream_slices(gpu, monkeypatch, T, shape):
 
 # The streamed GEMM's token groups at their edges (up to 8 tokens: hi and lo in
 # one MFMA; up to 16, 32 and 48), four- and eight-wave workgroups ("kr,rgw,nw":
-# quant blocks of a slice, units of 16 rows per wave, waves), one unsplit slice,
-# slices that end in a partial register set, waves past N.  Bound as in
+# quant blocks of a slice, units of 16 rows per wave, waves), one unsplit slice
+# (the widest a group takes, among them), slices that end in a partial register
+# set, waves past N.  (Products past the streamed lengths take the wide tile;
+# tests/test_prefill_dispatch.py holds the others to their cuts.)  Bound as in
 # test_prefill_wide_tiles: the activations enter at 22 (16) bits.
-@pytest.mark.parametrize("mode", [gh.QUANT_Q4, gh.QUANT_Q8, gh.QUANT_NONE])
-@pytest.mark.parametrize("T,N,K,cut", [
+STREAM_CUTS = [
     (1, 33, 128, "4,1,8"), (8, 200, 640, "12,1,4"), (8, 130, 1280, "40,2,4"), (9, 47, 640, "20,1,8"),
-    (16, 300, 2560, "80,1,8"), (15, 100, 1280, "40,1,4"), (17, 90, 1280, "20,3,4"),
-    (32, 140, 1280, "40,1,8"), (33, 70, 1024, "32,2,8"), (48, 260, 640, "16,1,4"),
-    (48, 50, 640, "20,1,8")])
+    (16, 300, 2432, "76,1,8"), (15, 100, 1280, "40,1,4"), (17, 90, 1280, "20,3,4"),
+    (32, 140, 1152, "36,1,8"), (33, 70, 1024, "32,2,8"), (40, 70, 896, "28,1,8"), (48, 260, 640, "16,1,4"),
+    (48, 50, 640, "20,1,8")]
+
+
+@pytest.mark.parametrize("mode", [gh.QUANT_Q4, gh.QUANT_Q8, gh.QUANT_NONE])
+@pytest.mark.parametrize("T,N,K,cut", STREAM_CUTS)
 def test_prefill_stream_cuts(gpu, monkeypatch, mode, T, N, K, cut):
     monkeypatch.setenv("GH_PF_STREAM", cut)
     rtol = 1e-3 if mode == gh.QUANT_NONE else 2e-5
