@@ -1,7 +1,9 @@
 // load_lds.h -- direct loads from memory to LDS: 16 bytes per lane from the
 // lane's address to LDS byte lds + 16 * lane (lds uniform).  They complete in
 // order with the wave's other loads and are waited for with vmcnt; the compiler
-// does not know of them, so the kernels write the waits out.
+// does not know of them, so the kernels write the waits out.  (It notes that m0 is
+// a reserved register: its own uses set m0 just ahead, and the clobber keeps them
+// from sharing a value across these.)
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

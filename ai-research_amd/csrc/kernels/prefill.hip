@@ -444,17 +444,20 @@ GH_GEMM_PAIR_W8(gh_pf_gateup_q4_m128_n64, Q4W, 128, 64, 1, true, _s_w8)
 // _bf16).  Operands as the tile GEMM's above; a block's sum is its hi
 // products, then its lo products (the streamed GEMM's order below).
 //
-// What bounds it: the matrix pipes and the power they draw.  A step of one
-// block of K is 2048 matrix cycles of a CU at TM = 4, BR = 256, and about
-// 1570 vector cycles (a scale FMA per result, the weights' unpacking); under
-// random data the chip runs these at 1.4-1.8 GHz (a register-only loop of the
-// same MFMA: 1.9-2.0 PFLOP/s, 1.65-1.85 for the 32x32x16 form, which is why
-// this one uses 16x16x32), so whatever else a step does costs time as power
-// even where it overlaps:
+// What bounds it: matrix and vector instructions, which overlap only in part, and
+// the power they draw.  A step of one block of K is 2048 matrix cycles of a CU at
+// TM = 4, BR = 256, and about 1570 vector cycles (a scale FMA per result, the
+// weights' unpacking).  Counters of the gate/up of 512 tokens: matrix pipes busy
+// 50% of the cycles, vector instructions beside them in 38% of those, waves
+// waiting 30%.  Under random data the chip runs these at 1.4-1.8 GHz (a
+// register-only loop of the same MFMA: 1.9-2.0 PFLOP/s, 1.65-1.85 for the 32x32x16
+// form, which is why this one uses 16x16x32), so whatever else a step does costs
+// time as power even where it overlaps:
 //  * operands go from memory to LDS directly (16 bytes per lane, no registers
 //    and no LDS store instructions).  The A rows are swizzled on the way, by
 //    permuting the lanes' source addresses within a row's 128 bytes, so that
-//    the operand reads are free of bank conflicts;
+//    the operand reads of 16 lanes (one g) meet no bank twice.  The counters
+//    still show 4 conflict cycles per LDS instruction, not taken apart yet;
 //  * quantized weights stay packed in LDS, four blocks of K (80 or 144 bytes
 //    of a row) at a time, and each wavefront unpacks the words of its rows as
 //    it reads them: a quarter (Q4) of the LDS bytes of fp16 weights;
@@ -478,8 +481,8 @@ GH_GEMM_PAIR_W8(gh_pf_gateup_q4_m128_n64, Q4W, 128, 64, 1, true, _s_w8)
 //
 // Measured, 12B gate/up of 512 tokens, tile GEMM -> this (the whole call, its
 // activation split included): Q4 281 -> 209 us (1160 TFLOP/s executed), Q8 297 ->
-// 219, bf16 269 -> 189.  Within a whole prompt's trace the Q4 kernel takes 224 us,
-// at a lower clock.  Timing-only copies took 11% less without the loads, 22%
+// 219, bf16 269 -> 189.  Within a whole prompt's trace the Q4 kernel alone
+// takes 212-221 us, at a lower clock.  Timing-only copies took 11% less without the loads, 22%
 // without the LDS reads of A as well.  The gate/up of 128 tokens (TM 2, BR 128,
 // which keeps K unsplit) 89 -> 73 us, of 64 tokens 61 -> 52 us.
 // ---------------------------------------------------------------------------

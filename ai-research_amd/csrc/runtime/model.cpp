@@ -1252,9 +1252,9 @@ gh_status prefill_batch(gh_model* m, const float* x, bool x_up, uint32_t T, cons
   // Grouped attention: the matrix-core kernel when every layer has head_dim
   // 256 and one G = nq / nkv dividing 16 (16 / G tokens per group) and the
   // batch has more than 64 tokens, else the 4-token kernel when every layer
-  // has G <= 2 and head_dim <= 256, else the per-token kernel.  The union of a group's lists keeps the order of first
-  // appearance; a list that names one slot twice keeps the per-token kernel
-  // (a union entry counts a slot once per token).
+  // has G <= 2 and head_dim <= 256, else the per-token kernel.  The union of a
+  // group's lists keeps the order of first appearance; a list that names one slot
+  // twice keeps the per-token kernel (a union entry counts a slot once per token).
   uint32_t gkind = 0, gtok = 0;
   {
     bool all256 = true, small = true, sameG = true;
@@ -1268,11 +1268,10 @@ gh_status prefill_batch(gh_model* m, const float* x, bool x_up, uint32_t T, cons
     }
     if (all256 && sameG && G0 >= 1 && G0 <= 16 && 16 % G0 == 0) {
       // up to 64 tokens the per-token kernel (one workgroup per kv head and
-      // token) is as fast or faster: 12B shape, 16 / 32 / 64 tokens
-      // 5.66 / 6.65 / 9.95 ms against 5.83 / 6.83 / 10.05 ms; at 96 the two
-      // tie and at 128 the matrix-core kernel leads (14.67 against 14.70 ms).
-      // GH_PF_ATTN_MFMA=1 (read per call) takes the matrix-core kernel for
-      // any batch.
+      // token) is as fast or faster: prompts of 16 / 32 / 48 / 64 tokens through
+      // eight layers of the 12B shape 851 / 1050 / 1278 / 1363 us against 869 /
+      // 1069 / 1282 / 1370.  GH_PF_ATTN_MFMA=1 (read per call) takes the
+      // matrix-core kernel for any batch.
       const char* fm = getenv("GH_PF_ATTN_MFMA");
       if (T > 64 || (fm && fm[0] == '1')) gkind = 2;
       gtok = 16 / G0;
