@@ -1041,6 +1041,9 @@ extern "C" __global__ __launch_bounds__(PF_NT) void gh_pf_splitk_k(const float* 
 // Q4 gate/up of 2 x 6144 x 2048, 33 tokens, is off by 1.52e-7, 1.63e-7 in chains of
 // a whole set, 1.65e-7 in slices of 16 blocks each one chain; the 12B gate/up of 16
 // tokens by 2.34e-7 with one chain per slice of 60.  It takes no measurable time.
+// bf16 keeps one chain per slice: its 16-bit activations are 20 times further off,
+// and a set's end then waits for its last MFMA (weights from memory, gate/up of 8
+// tokens: 52.8 us, 59.5 with a sum per set).
 //
 // AF (the o and down inputs, and the kernel-level f32 entry points): A comes
 // as f32 rows, and the staging splits each token's slice itself, with a
@@ -1326,7 +1329,7 @@ __device__ __forceinline__ void stream_gemm(const _Float16* __restrict__ Ax,
     float d[2][4];
     f32x4 acc[NG];
 #pragma unroll
-    for (int h = 0; h < NG; h++) acc[h] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int h = 0; h < NG; h++) acc[h] = F::kBf16 ? total[h] : f32x4{0.f, 0.f, 0.f, 0.f};
     read_a(x[0], 0);
     F::take(flat, 0, w, d[0]);
     b = F::half(w[0], uc);
@@ -1366,7 +1369,12 @@ __device__ __forceinline__ void stream_gemm(const _Float16* __restrict__ Ax,
       }
     }
 #pragma unroll
-    for (int h = 0; h < NG; h++) total[h] += acc[h];
+    for (int h = 0; h < NG; h++) {
+      if constexpr (F::kBf16)
+        total[h] = acc[h];
+      else
+        total[h] += acc[h];
+    }
   };
 
   for (uint32_t c = 0; c < nchunks; c += 2) {
