@@ -511,8 +511,10 @@ WideLds wide_lds_of(gh_quant_mode mode, uint32_t tm, uint32_t br) {
 // modes, 9 shapes of 2048 - 15360 rows by 1536 - 15360, 11 lengths of 49 - 512
 // tokens, up to 30 tiles and splits each): over 297 of them the tile taken is 1.3%
 // behind the best one in the mean and 19% at worst.  The 64- and 128-row tiles of
-// one K block per barrier take 1.21 times as long in the mean; they were ahead in 3
-// of 165 products (by 1 - 5%, 2944 x 9600 of 400 and 512 tokens).
+// one K block per barrier take 1.23 times as long in the mean; they were ahead in 1
+// of 165 products (by 1.7%, bf16 2944 x 9600 of 512 tokens).  Constants fitted to
+// products with their planes' sum (624 of 16 shapes, 1.1% behind) were worse in
+// whole prompts, whose norms add the planes: Q8 of 256 tokens 383 -> 398 us a layer.
 // GH_PF_WIDE="tm,nz,br" forces one.
 WideShape wide_shape(const gh_context* ctx, gh_quant_mode mode, bool pair, uint32_t T, uint32_t N,
                      uint32_t K) {
@@ -524,7 +526,7 @@ WideShape wide_shape(const gh_context* ctx, gh_quant_mode mode, bool pair, uint3
         ((r == 256 && t <= 4) || (r == 128 && t <= 3)))
       return WideShape{t, r, std::min(std::min(z, nq), 64u)};
   }
-  static const double step_us[2][4] = {{0.37, 0.55, 0.79, 0}, {0.75, 1.04, 1.27, 1.63}};
+  static const double step_cost[2][4] = {{0.37, 0.55, 0.79, 0}, {0.75, 1.04, 1.27, 1.63}};
   double least = 0;
   for (uint32_t br = 128; br <= 256; br += 128) {
     for (uint32_t tm = 1; tm <= (br == 128 ? 3u : 4u); tm++) {
@@ -535,7 +537,7 @@ WideShape wide_shape(const gh_context* ctx, gh_quant_mode mode, bool pair, uint3
       for (uint32_t nz = 1; nz <= std::max(1u, zmax); nz++) {
         const double load = (double)(tiles * nz) / cus;
         const double rounds = load <= 1 ? 1 : twice ? ceil(2 * load) / 2 : ceil(load);
-        double cost = rounds * (4.0 * ((nq + nz - 1) / nz) * step_us[br / 256][tm - 1] + 19);
+        double cost = rounds * (4.0 * ((nq + nz - 1) / nz) * step_cost[br / 256][tm - 1] + 19);
         if (nz > 1) cost += 1.5 + 1.03 * nz * (pair ? 2 : 1) * T * (double)N * 8 / 4e6;
         if (best.tm == 0 || cost < least) {
           least = cost;
